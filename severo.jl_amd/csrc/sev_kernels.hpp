@@ -429,7 +429,22 @@ struct KnnWork {
     DevBuf<uint64_t> skey64, skey64b;
     DevBuf<int32_t> cidx, ccnt, nfail, pidx, pcnt, perm, sval;
     DevBuf<int64_t> fail, fail2, qpad;
+    DevBuf<float> zs, piv;               // cell search: rows in slot order, pivots
+    DevBuf<int32_t> sval2, ccell, ctot;  // cell search: sorted ids, cell sizes, groups
+    DevBuf<int64_t> coff;
 };
+// ---- sev_knn_cell.hip ----------------------------------------------------
+// The exact kNN by a candidate search over cells of nearby points, which
+// skips the cells that lie beyond every query's k-th neighbour.  split: the
+// FP32 form (operands in two FP16 parts); otherwise one part, and -1 is
+// returned (nothing written) when the points have no clusters to skip.
+// Returns the rows without a certificate (their numbers in w.fail).
+constexpr int64_t kCellMinPoints = 4096;
+constexpr double kCellMaxShare = 0.4;
+bool knn_cell_fits(int64_t n, int64_t d, int64_t k);
+int64_t knn_cell(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
+                 bool split, KnnWork &w, int32_t *idx, float *dist, hipStream_t st);
+
 void knn_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
               int bf16, KnnWork &w, int32_t *idx, float *dist, hipStream_t st,
               int64_t *n_fallback);

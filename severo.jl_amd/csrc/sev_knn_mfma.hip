@@ -1151,12 +1151,22 @@ void cand_rerank(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, in
 
 template <int MODE, int KP, int QW, int KL, int KP32>
 void run_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
-              KnnWork &w, int32_t *idx, float *dist, hipStream_t st, int64_t *n_fallback) {
-    w.nfail.ensure(3);
+              KnnWork &w, int32_t *idx, float *dist, hipStream_t st, int64_t *n_fallback,
+              int64_t rows = -1) {
+    // all rows, or (rows >= 0) the first `rows` of w.fail
+    const int64_t *list = nullptr;
+    if (rows >= 0) {
+        w.fail2.ensure((size_t)rows);
+        SEV_HIP(hipMemcpyAsync(w.fail2.get(), w.fail.get(), sizeof(int64_t) * rows,
+                               hipMemcpyDeviceToDevice, st));
+        list = w.fail2.get();
+    }
+    w.nfail.ensure(4);
     w.fail.ensure((size_t)n);
     SEV_HIP(hipMemsetAsync(w.nfail.get(), 0, 3 * sizeof(int32_t), st));
-    cand_rerank<MODE, KP, QW, KL>(Z, n, d, ld, k, include_self, nullptr, n, w, idx, dist,
-                                  w.nfail.get(), w.fail.get(), st, nullptr, nullptr, true, 1);
+    cand_rerank<MODE, KP, QW, KL>(Z, n, d, ld, k, include_self, list, rows >= 0 ? rows : n, w, idx,
+                                  dist, w.nfail.get(), w.fail.get(), st, nullptr, nullptr, true,
+                                  1);
     int32_t nf = 0;
     SEV_HIP(hipMemcpyAsync(&nf, w.nfail.get(), sizeof nf, hipMemcpyDeviceToHost, st));
     SEV_HIP(hipStreamSynchronize(st));
@@ -1274,41 +1284,49 @@ void knn_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int i
     SEV_REQUIRE(k >= 1 && k <= kMaxK, "knn: k must be in [1, 64]");
     SEV_REQUIRE(d >= 1, "knn: d must be >= 1");
     SEV_REQUIRE(n < ((int64_t)1 << 31) - 256, "knn: at most 2^31 - 256 points");
+    int64_t rows = -1;
+    if (knn_cell_fits(n, d, k)) {
+        rows = knn_cell(Z, n, d, ld, k, include_self, !bf16, w, idx, dist, st);
+        if (rows == 0) {
+            if (n_fallback) *n_fallback = 0;
+            return;
+        }
+    }
     if (bf16) {
         SEV_REQUIRE(d + 2 <= 128, "knn: BF16 form supports d <= 126");
         if (k <= 24 && d + 2 <= 64 && d + 1 <= 52)
-            run_mfma<1, 64, 2, 32, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback);
+            run_mfma<1, 64, 2, 32, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback, rows);
         else if (k <= 40 && d + 2 <= 64 && d + 1 <= 52)
-            run_mfma<1, 64, 2, 48, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback);
+            run_mfma<1, 64, 2, 48, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback, rows);
         else if (k <= 24 && d + 2 <= 64)
             run_mfma<1, 64, 2, 32, 128>(Z, n, d, ld, k, include_self, w, idx, dist, st,
-                                        n_fallback);
+                                        n_fallback, rows);
         else if (k <= 24)
             run_mfma<1, 128, 2, 32, 128>(Z, n, d, ld, k, include_self, w, idx, dist, st,
-                                         n_fallback);
+                                         n_fallback, rows);
         else if (d + 2 <= 64 && d + 1 <= 52)
             run_mfma<1, 64, 1, 64, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st,
-                                       n_fallback);
+                                       n_fallback, rows);
         else if (d + 2 <= 64)
-            run_mfma<1, 64, 1, 64, 0>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback);
+            run_mfma<1, 64, 1, 64, 0>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback, rows);
         else
-            run_mfma<1, 128, 1, 64, 0>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback);
+            run_mfma<1, 128, 1, 64, 0>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback, rows);
     } else {
         SEV_REQUIRE(d + 1 <= 128, "knn: FP32 MFMA form supports d <= 127");
         if (d + 1 <= 52) {
             if (k <= 24)
                 run_mfma<0, 52, 2, 32, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st,
-                                           n_fallback);
+                                           n_fallback, rows);
             else if (k <= 40)
                 run_mfma<0, 52, 2, 48, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st,
-                                           n_fallback);
+                                           n_fallback, rows);
             else
                 run_mfma<0, 52, 1, 64, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st,
-                                           n_fallback);
+                                           n_fallback, rows);
         } else {
             if (k <= 24) {
                 run_mfma<0, 128, 1, 32, 128>(Z, n, d, ld, k, include_self, w, idx, dist, st,
-                                             n_fallback);
+                                             n_fallback, rows);
             } else {
                 // wide rows with long lists exceed the LDS budget: exhaustive
                 knn_exact<float>(Z, n, d, ld, k, include_self, nullptr, n, idx, dist, st);

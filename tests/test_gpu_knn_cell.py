@@ -1,0 +1,42 @@
+"""The neighbour search over cells against the oracle's exhaustive search, bit
+for bit: clustered points at the edges of the search's operand widths, group
+and cell sizes, with rare clusters, duplicates and points far off."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _points(n, d, groups, seed, spread=8.0, dup=0):
+    rng = np.random.default_rng(seed)
+    centre = rng.normal(0, spread, (groups, d))
+    lab = np.minimum(rng.geometric(2.0 / groups, n) - 1, groups - 1)  # uneven, some rare
+    X = (centre[lab] + rng.normal(0, 1.0, (n, d))).astype(np.float32)
+    if dup:
+        X[rng.integers(0, n, dup)] = X[rng.integers(0, n, dup)]
+    return np.asfortranarray(X)
+
+
+@pytest.mark.parametrize("include_self", [True, False])
+@pytest.mark.parametrize("n,d,k,groups,dup",
+                         [(4096, 20, 10, 12, 0), (4097, 21, 5, 7, 200), (6001, 31, 24, 20, 0),
+                          (9000, 41, 30, 9, 0), (5000, 52, 20, 30, 500), (4999, 63, 1, 5, 0),
+                          (12345, 50, 20, 40, 0), (7000, 3, 15, 6, 0)])
+def test_cells_bit_exact(sev, orc, n, d, k, groups, dup, include_self):
+    X = _points(n, d, groups, seed=n + d, dup=dup)
+    ridx, rdist = orc.knn(X, k, include_self=include_self)
+    for precision in ("fp32", "bf16"):
+        idx, dist = sev.ann(X, k, include_self=include_self, precision=precision)
+        assert np.array_equal(idx, ridx), precision
+        assert np.array_equal(dist, rdist), precision
+
+
+def test_cells_degenerate(sev, orc):
+    """Identical points, one point far from all others, all-zero columns."""
+    X = _points(5000, 12, 4, seed=3)
+    X[:3000] = X[0]
+    X[4999] = 1e4
+    X[:, 5] = 0.0
+    idx, dist = sev.ann(X, 15, precision="fp32")
+    ridx, rdist = orc.knn(X, 15)
+    assert np.array_equal(idx, ridx) and np.array_equal(dist, rdist)
