@@ -25,6 +25,13 @@
 // normal range are taken as zero, so their treatment by the MFMA does not
 // matter.
 //
+// Measured, k = 20: 1,000,000 x 50, 40 clusters, one part: 526 -> 73 ms (65 of
+// them k_knn_cell); 100,000 x 50, 24 clusters, two parts: 27.3 -> 3.6 ms;
+// 5,000 x 50: 1.68 -> 0.66 ms.  Without clusters nothing is skipped and the two
+// sweeps cost more than the one with insertion (1,000,000 Gaussian points: 165
+// ms by sev_knn_mfma.hip), so the 16-bit form keeps that search there; the FP32
+// form is faster this way in either case.
+//
 // Two sweeps and no insertion.  The largest score of each of the 64 residues
 // of the tile position is kept in registers over a sweep; the r-th largest of
 // the 64 is reached by r candidates.  A sweep over the nearest groups in slot
@@ -32,6 +39,12 @@
 // gives the final threshold, and a second one appends what exceeds it: about
 // 64 ln(64 / (64 - r)) candidates, 40 at r = 30 for k = 20.  Sorted insertion of each
 // passing pair, one at a time, had cost more than the products.
+//
+// A block holds 128 queries (4 wavefronts of 32) and 64-candidate tiles in
+// two LDS buffers: 80 KB at KP = 160, so two blocks share a compute unit, three
+// at KP <= 64.  Bound: the candidate rows of the needed groups, which mostly
+// come from beyond L2 (1.3 us per tile and block at KP = 160, 0.27 us of them
+// MFMA).
 #include "sev_kernels.hpp"
 
 #include <hipcub/hipcub.hpp>

@@ -40,3 +40,19 @@ def test_cells_degenerate(sev, orc):
     idx, dist = sev.ann(X, 15, precision="fp32")
     ridx, rdist = orc.knn(X, 15)
     assert np.array_equal(idx, ridx) and np.array_equal(dist, rdist)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,d,k", [(70, 5, 63), (65, 2, 64), (255, 7, 20), (257, 50, 1),
+                                   (4095, 9, 30), (4400, 17, 12)])
+def test_exhaustive_head_bound(sev, orc, dtype, n, d, k):
+    """The exhaustive search at the edges of its tiles and of the head sweep
+    that bounds the k-th neighbour, with many equal distances."""
+    X = _points(n, d, 3, seed=n + k, dup=n // 3).astype(dtype)
+    X[: n // 4] = np.round(X[: n // 4])
+    for include_self in (True, False):
+        kk = min(k, n if include_self else n - 1)
+        idx, dist = sev.ann(np.asfortranarray(X), kk, include_self=include_self,
+                            precision="exact")
+        ridx, rdist = orc.knn(np.asfortranarray(X), kk, include_self=include_self)
+        assert np.array_equal(idx, ridx) and np.array_equal(dist, rdist)
