@@ -429,7 +429,8 @@ struct KnnWork {
     DevBuf<uint64_t> skey64, skey64b;
     DevBuf<int32_t> cidx, ccnt, nfail, pidx, pcnt, perm, sval;
     DevBuf<int64_t> fail, fail2, qpad;
-    DevBuf<float> zs, piv;               // cell search: rows in slot order, pivots
+    DevBuf<unsigned char> zrb, zs;       // cell search: rows, rows in slot order
+    DevBuf<float> piv;                   // cell search: pivots, sample
     DevBuf<int32_t> sval2, ccell, ctot;  // cell search: sorted ids, cell sizes, groups
     DevBuf<int64_t> coff;
 };
@@ -441,9 +442,17 @@ struct KnnWork {
 // Returns the rows without a certificate (their numbers in w.fail).
 constexpr int64_t kCellMinPoints = 4096;
 constexpr double kCellMaxShare = 0.4;
+// FP64 points: by cells above these sizes (one call on host arrays: 15,000 x
+// 50: 2.6 ms, exhaustively 3.2; 10,000 x 50: 2.3 against 1.9; 20,011 x 15: 1.6
+// against 1.8; 15,000 x 15: 1.4 against 1.2)
+inline bool knn_cell_f64_pays(int64_t n, int64_t d) { return n > 18000 || n * d > 600000; }
 bool knn_cell_fits(int64_t n, int64_t d, int64_t k);
-int64_t knn_cell(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
-                 bool split, KnnWork &w, int32_t *idx, float *dist, hipStream_t st);
+template <class T>
+int64_t knn_cell(const T *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
+                 bool split, KnnWork &w, int32_t *idx, T *dist, hipStream_t st);
+// FP64 points (the FP64 definition); rows without a certificate exhaustively.
+void knn_cell_f64(const double *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
+                  KnnWork &w, int32_t *idx, double *dist, hipStream_t st, int64_t *n_fallback);
 
 void knn_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
               int bf16, KnnWork &w, int32_t *idx, float *dist, hipStream_t st,

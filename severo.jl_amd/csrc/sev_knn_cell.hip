@@ -52,6 +52,7 @@
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace sev {
@@ -96,9 +97,10 @@ __device__ __forceinline__ float point_scale(unsigned n2) {
 }
 
 // Zr[i*d + t] = Z[t*ld + i], 64 points per block through LDS; n2 = max |z|^2
+template <class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_rows(const float *Z, int64_t n, int d, int64_t ld, float *Zr, unsigned *n2) {
-    __shared__ float s[kWave * 65];
+k_cell_rows(const T *Z, int64_t n, int d, int64_t ld, T *Zr, unsigned *n2) {
+    __shared__ T s[kWave * 65];
     __shared__ float nn[kNW][kWave];
     const int64_t i0 = (int64_t)blockIdx.x * kWave;
     const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
@@ -106,9 +108,9 @@ k_cell_rows(const float *Z, int64_t n, int d, int64_t ld, float *Zr, unsigned *n
     float a = 0.0f;
     for (int t = w; t < d; t += kNW)
         if (lane < nr) {
-            const float z = Z[(int64_t)t * ld + i0 + lane];
+            const T z = Z[(int64_t)t * ld + i0 + lane];
             s[lane * (d + 1) + t] = z;
-            a = fmaf(z, z, a);
+            a = fmaf((float)z, (float)z, a);
         }
     nn[w][lane] = a;
     __syncthreads();
@@ -123,20 +125,22 @@ k_cell_rows(const float *Z, int64_t n, int d, int64_t ld, float *Zr, unsigned *n
 }
 
 // piv[m*kPivLd + t] = coordinates of the point (m * n) / M, zero padded
+template <class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_pivots(const float *Zr, int64_t n, int d, int M, float *piv) {
+k_cell_pivots(const T *Zr, int64_t n, int d, int M, float *piv) {
     for (int e = blockIdx.x * kBlock + threadIdx.x; e < M * kPivLd; e += gridDim.x * kBlock) {
         const int m = e / kPivLd, t = e % kPivLd;
-        piv[e] = t < d ? Zr[((int64_t)m * n / M) * d + t] : 0.0f;
+        piv[e] = t < d ? (float)Zr[((int64_t)m * n / M) * d + t] : 0.0f;
     }
 }
 
 // S[t*ns + i] = coordinates of the point (i * n) / ns
+template <class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_sample(const float *Zr, int64_t n, int d, int ns, float *S) {
+k_cell_sample(const T *Zr, int64_t n, int d, int ns, float *S) {
     for (int e = blockIdx.x * kBlock + threadIdx.x; e < ns * d; e += gridDim.x * kBlock) {
         const int t = e / ns, i = e % ns;
-        S[e] = Zr[((int64_t)i * n / ns) * d + t];
+        S[e] = (float)Zr[((int64_t)i * n / ns) * d + t];
     }
 }
 
@@ -187,13 +191,14 @@ k_cell_means(const float *S, int ns, int d, const uint32_t *cell, float *piv, fl
 // the distance of the nearest one, for each of kTestQueries sampled queries.
 // Within one Gaussian blob all distances are alike (a share near 1); among
 // clusters the share is that of the query's own and the overlapping ones.
+template <class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_test(const float *Zr, int64_t n, int d, const float *piv, int *share) {
+k_cell_test(const T *Zr, int64_t n, int d, const float *piv, int *share) {
     __shared__ float q[64];
     __shared__ float best[kNW];
     __shared__ int cnt;
     const int64_t i = ((int64_t)blockIdx.x * n) / kTestQueries + n / (2 * kTestQueries);
-    if (threadIdx.x < d) q[threadIdx.x] = Zr[(i < n ? i : n - 1) * d + threadIdx.x];
+    if (threadIdx.x < d) q[threadIdx.x] = (float)Zr[(i < n ? i : n - 1) * d + threadIdx.x];
     if (threadIdx.x == 0) cnt = 0;
     __syncthreads();
     float D[kTestPivots / kBlock];
@@ -260,9 +265,9 @@ k_cell_order(const float *piv, const float *half, int M, int d, float *out, floa
 // Nearest pivot of each point (any choice is correct: it only shapes the
 // cells); counts per cell when asked for.  The pivots are read at uniform
 // addresses, so they reach the FMAs as scalar operands.
-template <int DP>
+template <int DP, class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_assign(const float *Z, int64_t n, int d, int64_t ld, const float *__restrict__ piv,
+k_cell_assign(const T *Z, int64_t n, int d, int64_t ld, const float *__restrict__ piv,
               const float *__restrict__ half, int M, uint32_t *cell, int32_t *id, int32_t *cnt) {
     __shared__ int lc[kMaxPivots];
     if (cnt)
@@ -270,7 +275,7 @@ k_cell_assign(const float *Z, int64_t n, int d, int64_t ld, const float *__restr
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     float z[DP];
 #pragma unroll
-    for (int t = 0; t < DP; ++t) z[t] = (t < d && i < n) ? -Z[(int64_t)t * ld + i] : 0.0f;
+    for (int t = 0; t < DP; ++t) z[t] = (t < d && i < n) ? -(float)Z[(int64_t)t * ld + i] : 0.0f;
     float best = __builtin_huge_valf();
     int bm = 0;
     for (int m = 0; m < M; ++m) {
@@ -337,10 +342,10 @@ k_cell_slots(const uint32_t *scell, const int32_t *sid, int64_t n, const int64_t
 // centre rows [h, n1, n2, n3], n1 + n2 + n3 = -|y|^2 / 2; two parts: [h, l, h,
 // 1, 1, 1] and [h, h, l, n1, n2, n3].  gmax: [0] max |y|^2 and [1] max error over
 // the points, [2] max |y|^2 over the means, [3] max |z|^2 unscaled.
-template <int KP, bool SPLIT>
+template <int KP, bool SPLIT, class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_prep(const float *Zr, int d, const int32_t *perm, const int *tot, uint16_t *zq,
-            uint16_t *zc, uint16_t *zb, float *Rb, float *Zs, float *nhat, float *eps,
+k_cell_prep(const T *Zr, int d, const int32_t *perm, const int *tot, uint16_t *zq,
+            uint16_t *zc, uint16_t *zb, float *Rb, T *Zs, float *nhat, float *eps,
             unsigned *gmax) {
     __shared__ float zt[kGrp * 65];
     __shared__ uint16_t nc[kGrp + 1][4];
@@ -365,9 +370,9 @@ k_cell_prep(const float *Zr, int d, const int32_t *perm, const int *tot, uint16_
     __syncthreads();
     for (int e = tid; e < kGrp * d; e += kBlock) {
         const int r = e / d, t = e - r * d;
-        const float z = ids[r] >= 0 ? Zr[(int64_t)ids[r] * d + t] : 0.0f;
+        const T z = ids[r] >= 0 ? Zr[(int64_t)ids[r] * d + t] : T(0);
         Zs[s0 * d + e] = z;
-        zt[r * ldz + t] = z * sc;
+        zt[r * ldz + t] = (float)(z * (T)sc);
     }
     __syncthreads();
     if (tid < d) {
@@ -388,7 +393,10 @@ k_cell_prep(const float *Zr, int d, const int32_t *perm, const int *tot, uint16_
             double y = (double)h2f(h);
             if constexpr (SPLIT) y += (double)h2f(f2h(z - h2f(h)));
             nn += y * y;
-            ee += (y - (double)z) * (y - (double)z);
+            double x = (double)z;
+            if constexpr (sizeof(T) == 8)  // against the double, not its FP32 rounding
+                if (tid < kGrp) x = (double)Zs[(s0 + tid) * d + t] * (double)sc;
+            ee += (y - x) * (y - x);
             a = fmaf(z - mean[t], z - mean[t], a);
         }
         const bool live = tid == kGrp || ids[tid] >= 0;
@@ -465,7 +473,11 @@ k_cell_prep(const float *Zr, int d, const int32_t *perm, const int *tot, uint16_
         atomicMax(&gmax[0], max(red[0][0], red[0][1]));
         atomicMax(&gmax[1], max(red[1][0], red[1][1]));
         atomicMax(&gmax[2], __float_as_uint(nf));
-        Rb[g] = (__uint_as_float(max(red[2][0], red[2][1])) + ef) * (1.0f + 1e-5f) + 1e-30f;
+        float r = __uint_as_float(max(red[2][0], red[2][1])) + ef;
+        // the radius was taken of the FP32 roundings of the doubles
+        if constexpr (sizeof(T) == 8)
+            r += 1.2e-7f * sqrtf(__uint_as_float(max(red[0][0], red[0][1])));
+        Rb[g] = r * (1.0f + 1e-5f) + 1e-30f;
     }
 }
 
@@ -803,11 +815,12 @@ k_knn_cell(CellArgs a) {
 
 // Exact distances of a query's candidates (unscaled rows), the k smallest under (distance,
 // index), and the certificate of sev_knn_mfma.hip; one wavefront per slot.
+template <class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_rerank(const float *Zs, const int32_t *perm, const int *tot, int d, int k,
+k_cell_rerank(const T *Zs, const int32_t *perm, const int *tot, int d, int k,
               const int32_t *cidx, const int32_t *ccnt, const float *cthr, const float *nhat,
               const float *eps, const unsigned *gmax, double eta, double spec, int32_t *oidx,
-              float *odist, int32_t *nfail, int64_t *fail) {
+              T *odist, int32_t *nfail, int64_t *fail) {
     const int lane = lane_id();
     const int64_t s = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
     if (s >= (int64_t)tot[0] * kGrp) return;
@@ -815,26 +828,27 @@ k_cell_rerank(const float *Zs, const int32_t *perm, const int *tot, int d, int k
     if (q < 0) return;
     const int cnt = ccnt[s];
     const int32_t c = lane < cnt && cnt <= kCap ? cidx[s * kCap + lane] : -1;
-    float D = __builtin_huge_valf();
+    T D = (T)__builtin_huge_valf();
     int32_t ci = INT_MAX;
     if (c >= 0) {
+        typedef T T2 __attribute__((ext_vector_type(2)));
         ci = perm[c];
-        const float *zq = Zs + s * d, *zc = Zs + (int64_t)c * d;
-        float acc = 0.0f;
-        if ((d & 1) == 0) {
-            const float2 *q2 = (const float2 *)zq, *c2 = (const float2 *)zc;
+        const T *zq = Zs + s * d, *zc = Zs + (int64_t)c * d;
+        T acc = 0;
+        if ((d & 1) == 0) {  // rows start at a multiple of two values
+            const T2 *q2 = (const T2 *)zq, *c2 = (const T2 *)zc;
 #pragma unroll 4
             for (int t = 0; t < d / 2; ++t) {
-                const float2 x = q2[t], y = c2[t];
-                const float d0 = x.x - y.x;
+                const T2 x = q2[t], y = c2[t];
+                const T d0 = x[0] - y[0];
                 acc = acc + d0 * d0;
-                const float d1 = x.y - y.y;
+                const T d1 = x[1] - y[1];
                 acc = acc + d1 * d1;
             }
         } else {
 #pragma unroll 4
             for (int t = 0; t < d; ++t) {
-                const float x = zq[t] - zc[t];
+                const T x = zq[t] - zc[t];
                 acc = acc + x * x;
             }
         }
@@ -842,7 +856,7 @@ k_cell_rerank(const float *Zs, const int32_t *perm, const int *tot, int d, int k
     }
     for (int size = 2; size <= kWave; size <<= 1)
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            const float oD = __shfl_xor(D, stride, kWave);
+            const T oD = __shfl_xor(D, stride, kWave);
             const int32_t oc = __shfl_xor(ci, stride, kWave);
             const bool up = (lane & size) == 0, lower = (lane & stride) == 0;
             const bool less = oD < D || (oD == D && oc < ci);
@@ -852,7 +866,7 @@ k_cell_rerank(const float *Zs, const int32_t *perm, const int *tot, int d, int k
                 ci = oc;
             }
         }
-    const float Dk = __shfl(D, k - 1, kWave);
+    const T Dk = __shfl(D, k - 1, kWave);
     const double nq = (double)nhat[s];
     const double dt = nq - 2.0 * (double)cthr[s];
     const double lb2 = dt * (1.0 - 0x1p-21) -
@@ -865,16 +879,16 @@ k_cell_rerank(const float *Zs, const int32_t *perm, const int *tot, int d, int k
     if (ok) {
         if (lane < k) {
             oidx[(int64_t)q * k + lane] = ci;
-            odist[(int64_t)q * k + lane] = sqrtf(D);
+            odist[(int64_t)q * k + lane] = sqrt(D);
         }
     } else if (lane == 0) {
         fail[atomicAdd(nfail, 1)] = q;
     }
 }
 
-template <int KP, bool SPLIT>
+template <int KP, bool SPLIT, class T>
 void run_cell(int64_t n, int64_t d, int64_t k, int include_self, int M, KnnWork &w, int32_t *idx,
-              float *dist, hipStream_t st) {
+              T *dist, hipStream_t st) {
     const int64_t ngb = ceil_div(n, (int64_t)kGrp) + M;  // at least the groups in use
     const int64_t ns = ngb * kGrp;
     const int64_t ngt = ceil_div(ngb, (int64_t)kCT) * kCT;
@@ -882,7 +896,9 @@ void run_cell(int64_t n, int64_t d, int64_t k, int include_self, int M, KnnWork 
     w.zc.ensure((size_t)ns * KP * 2);
     w.zcp.ensure((size_t)ngt * KP * 2);
     w.scf.ensure((size_t)ngt);
-    w.zs.ensure((size_t)(ns * d));
+    w.zs.ensure((size_t)(ns * d) * sizeof(T));
+    const T *zr = (const T *)w.zrb.get();
+    T *zs = (T *)w.zs.get();
     w.nhat.ensure((size_t)ns);
     w.eps.ensure((size_t)ns);
     w.cidx.ensure((size_t)ns * kCap);
@@ -891,10 +907,10 @@ void run_cell(int64_t n, int64_t d, int64_t k, int include_self, int M, KnnWork 
     const int *tot = w.ctot.get();
     {
         ProfScope ps("knn_prep", st, 8.0 * n * d + 4.0 * n * KP);
-        hipLaunchKernelGGL((k_cell_prep<KP, SPLIT>), dim3((unsigned)ngt), dim3(kBlock), 0, st, w.zr.get(),
+        hipLaunchKernelGGL((k_cell_prep<KP, SPLIT, T>), dim3((unsigned)ngt), dim3(kBlock), 0, st, zr,
                            (int)d, w.perm.get(), tot, (uint16_t *)w.zq.get(),
                            (uint16_t *)w.zc.get(), (uint16_t *)w.zcp.get(), w.scf.get(),
-                           w.zs.get(), w.nhat.get(), w.eps.get(), w.gmax.get());
+                           zs, w.nhat.get(), w.eps.get(), w.gmax.get());
         SEV_LAUNCH_CHECK();
     }
     CellArgs a;
@@ -915,7 +931,7 @@ void run_cell(int64_t n, int64_t d, int64_t k, int include_self, int M, KnnWork 
     // FP32 accumulation over KP terms, the dropped l.l' (2^-22) and the
     // three-part norm
     a.eta = 4.0 * (KP + 2) * 0x1p-24 + 0x1p-20;
-    a.spec = pow(1.0 - 0x1p-24, (double)(d + 3));
+    a.spec = pow(1.0 - (sizeof(T) == 4 ? 0x1p-24 : 0x1p-53), (double)(d + 3));
     a.cidx = w.cidx.get();
     a.ccnt = w.ccnt.get();
     a.cthr = w.cthr.get();
@@ -929,8 +945,8 @@ void run_cell(int64_t n, int64_t d, int64_t k, int include_self, int M, KnnWork 
         SEV_LAUNCH_CHECK();
     }
     ProfScope ps("knn_rerank", st, (double)n * (kCap * 0.6) * (4.0 + 4.0 * d));
-    hipLaunchKernelGGL(k_cell_rerank, dim3((unsigned)ceil_div(ns * kWave, (int64_t)kBlock)),
-                       dim3(kBlock), 0, st, w.zs.get(), w.perm.get(), tot, (int)d, (int)k,
+    hipLaunchKernelGGL(k_cell_rerank<T>, dim3((unsigned)ceil_div(ns * kWave, (int64_t)kBlock)),
+                       dim3(kBlock), 0, st, (const T *)zs, w.perm.get(), tot, (int)d, (int)k,
                        w.cidx.get(), w.ccnt.get(), w.cthr.get(), w.nhat.get(), w.eps.get(),
                        w.gmax.get(), a.eta, a.spec, idx, dist, w.nfail.get(), w.fail.get());
     SEV_LAUNCH_CHECK();
@@ -945,13 +961,15 @@ bool knn_cell_fits(int64_t n, int64_t d, int64_t k) {
            d <= 63;
 }
 
-int64_t knn_cell(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
-                 bool split, KnnWork &w, int32_t *idx, float *dist, hipStream_t st) {
+template <class T>
+int64_t knn_cell(const T *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
+                 bool split, KnnWork &w, int32_t *idx, T *dist, hipStream_t st) {
     // cells of 1024 to 2048 points (smaller ones below 16,384 points)
     int M = 16;
     while (M < kMaxPivots && (int64_t)M * 1024 < n) M <<= 1;
     const int nsam = (int)std::min<int64_t>(n, kSample);
-    w.zr.ensure((size_t)(n * d));
+    w.zrb.ensure((size_t)(n * d) * sizeof(T));
+    T *zr = (T *)w.zrb.get();
     w.piv.ensure((size_t)(kTestPivots * kPivLd * 2 + 2 * kMaxPivots + kSample * 64));
     w.ctot.ensure(1);
     w.gmax.ensure(4);
@@ -959,15 +977,15 @@ int64_t knn_cell(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, in
           *half = pivo + kTestPivots * kPivLd, *halfo = half + kMaxPivots,
           *sam = halfo + kMaxPivots;
     SEV_HIP(hipMemsetAsync(w.gmax.get(), 0, 4 * sizeof(unsigned), st));
-    hipLaunchKernelGGL(k_cell_rows, dim3((unsigned)ceil_div(n, (int64_t)kWave)), dim3(kBlock), 0,
-                       st, Z, n, (int)d, ld, w.zr.get(), w.gmax.get() + 3);
+    hipLaunchKernelGGL(k_cell_rows<T>, dim3((unsigned)ceil_div(n, (int64_t)kWave)), dim3(kBlock), 0,
+                       st, Z, n, (int)d, ld, zr, w.gmax.get() + 3);
     SEV_LAUNCH_CHECK();
     if (!split) {
         w.ccnt.ensure((size_t)std::max<int64_t>(n, kTestQueries));
-        hipLaunchKernelGGL(k_cell_pivots, dim3(64), dim3(kBlock), 0, st, w.zr.get(), n, (int)d,
+        hipLaunchKernelGGL(k_cell_pivots<T>, dim3(64), dim3(kBlock), 0, st, zr, n, (int)d,
                            kTestPivots, piv);
         SEV_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_cell_test, dim3(kTestQueries), dim3(kBlock), 0, st, w.zr.get(), n,
+        hipLaunchKernelGGL(k_cell_test<T>, dim3(kTestQueries), dim3(kBlock), 0, st, zr, n,
                            (int)d, piv, w.ccnt.get());
         SEV_LAUNCH_CHECK();
         std::vector<int32_t> share(kTestQueries);
@@ -990,12 +1008,13 @@ int64_t knn_cell(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, in
         w.perm.ensure((size_t)ns);
         SEV_HIP(hipMemsetAsync(w.ccell.get(), 0, sizeof(int32_t) * kMaxPivots, st));
         SEV_HIP(hipMemsetAsync(w.perm.get(), 0xFF, sizeof(int32_t) * (size_t)ns, st));
-        auto assign = [&](const float *X, int64_t nx, int64_t lx, const float *pv, const float *hv,
+        auto assign = [&](const auto *X, int64_t nx, int64_t lx, const float *pv, const float *hv,
                           uint32_t *cell, int32_t *id, int32_t *cnt) {
             auto go = [&](auto dp) {
                 constexpr int DP = decltype(dp)::value;
-                hipLaunchKernelGGL(k_cell_assign<DP>, dim3((unsigned)ceil_div(nx, (int64_t)kBlock)),
-                                   dim3(kBlock), 0, st, X, nx, (int)d, lx, pv, hv, M, cell, id,
+                typedef std::remove_const_t<std::remove_pointer_t<decltype(X)>> TX;
+                hipLaunchKernelGGL((k_cell_assign<DP, TX>),
+                                   dim3((unsigned)ceil_div(nx, (int64_t)kBlock)), dim3(kBlock), 0, st, X, nx, (int)d, lx, pv, hv, M, cell, id,
                                    cnt);
             };
             if (d <= 16)
@@ -1008,15 +1027,15 @@ int64_t knn_cell(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, in
                 go(std::integral_constant<int, 64>());
             SEV_LAUNCH_CHECK();
         };
-        hipLaunchKernelGGL(k_cell_pivots, dim3(64), dim3(kBlock), 0, st, w.zr.get(), n, (int)d, M,
+        hipLaunchKernelGGL(k_cell_pivots<T>, dim3(64), dim3(kBlock), 0, st, zr, n, (int)d, M,
                            piv);
         hipLaunchKernelGGL(k_cell_half, dim3((unsigned)ceil_div((int64_t)M, (int64_t)kBlock)),
                            dim3(kBlock), 0, st, piv, M, half);
-        hipLaunchKernelGGL(k_cell_sample, dim3(256), dim3(kBlock), 0, st, w.zr.get(), n, (int)d,
+        hipLaunchKernelGGL(k_cell_sample<T>, dim3(256), dim3(kBlock), 0, st, zr, n, (int)d,
                            nsam, sam);
         SEV_LAUNCH_CHECK();
         for (int it = 0; it < 2; ++it) {
-            assign(sam, nsam, nsam, piv, half, w.skey2.get(), nullptr, nullptr);
+            assign((const float *)sam, nsam, nsam, piv, half, w.skey2.get(), nullptr, nullptr);
             hipLaunchKernelGGL(k_cell_means, dim3((unsigned)M), dim3(kBlock), 0, st, sam, nsam,
                                (int)d, w.skey2.get(), piv, half);
             SEV_LAUNCH_CHECK();
@@ -1049,28 +1068,41 @@ int64_t knn_cell(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, in
     if (split) {
         const int64_t cols = 3 * d + 3;
         if (cols <= 64)
-            run_cell<64, true>(n, d, k, include_self, M, w, idx, dist, st);
+            run_cell<64, true, T>(n, d, k, include_self, M, w, idx, dist, st);
         else if (cols <= 96)
-            run_cell<96, true>(n, d, k, include_self, M, w, idx, dist, st);
+            run_cell<96, true, T>(n, d, k, include_self, M, w, idx, dist, st);
         else if (cols <= 128)
-            run_cell<128, true>(n, d, k, include_self, M, w, idx, dist, st);
+            run_cell<128, true, T>(n, d, k, include_self, M, w, idx, dist, st);
         else if (cols <= 160)
-            run_cell<160, true>(n, d, k, include_self, M, w, idx, dist, st);
+            run_cell<160, true, T>(n, d, k, include_self, M, w, idx, dist, st);
         else
-            run_cell<192, true>(n, d, k, include_self, M, w, idx, dist, st);
+            run_cell<192, true, T>(n, d, k, include_self, M, w, idx, dist, st);
     } else {
         const int64_t cols = d + 3;
         if (cols <= 32)
-            run_cell<32, false>(n, d, k, include_self, M, w, idx, dist, st);
+            run_cell<32, false, T>(n, d, k, include_self, M, w, idx, dist, st);
         else if (cols <= 64)
-            run_cell<64, false>(n, d, k, include_self, M, w, idx, dist, st);
+            run_cell<64, false, T>(n, d, k, include_self, M, w, idx, dist, st);
         else
-            run_cell<96, false>(n, d, k, include_self, M, w, idx, dist, st);
+            run_cell<96, false, T>(n, d, k, include_self, M, w, idx, dist, st);
     }
     int32_t nf = 0;
     SEV_HIP(hipMemcpyAsync(&nf, w.nfail.get(), sizeof nf, hipMemcpyDeviceToHost, st));
     SEV_HIP(hipStreamSynchronize(st));
     return nf;
+}
+
+template int64_t knn_cell<float>(const float *, int64_t, int64_t, int64_t, int64_t, int, bool,
+                                 KnnWork &, int32_t *, float *, hipStream_t);
+
+// FP64 points: their FP32 roundings in two parts propose the candidates (the
+// rounding is part of each point's operand error), the exact FP64 distances
+// rank them.
+void knn_cell_f64(const double *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
+                  KnnWork &w, int32_t *idx, double *dist, hipStream_t st, int64_t *n_fallback) {
+    const int64_t nf = knn_cell<double>(Z, n, d, ld, k, include_self, true, w, idx, dist, st);
+    if (nf > 0) knn_exact_rows<double>(Z, n, d, ld, k, include_self, w.fail.get(), nf, idx, dist, st);
+    if (n_fallback) *n_fallback = nf;
 }
 
 }  // namespace sev

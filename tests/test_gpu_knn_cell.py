@@ -31,6 +31,20 @@ def test_cells_bit_exact(sev, orc, n, d, k, groups, dup, include_self):
         assert np.array_equal(dist, rdist), precision
 
 
+@pytest.mark.parametrize("include_self", [True, False])
+@pytest.mark.parametrize("n,d,k,spread", [(18001, 4, 10, 8.0), (12000, 51, 15, 1e-3),
+                                          (12100, 50, 30, 1e6)])
+def test_cells_fp64_bit_exact(sev, orc, n, d, k, spread, include_self):
+    """FP64 points, among them clusters so tight or so far from the origin
+    that their FP32 roundings coincide (those rows are searched exhaustively)."""
+    rng = np.random.default_rng(n)
+    X = np.asfortranarray(_points(n, d, 15, seed=k, spread=spread).astype(np.float64) +
+                          rng.normal(0, 1e-3, (n, d)))
+    idx, dist = sev.ann(X, k, include_self=include_self)
+    ridx, rdist = orc.knn(X, k, include_self=include_self)
+    assert np.array_equal(idx, ridx) and np.array_equal(dist, rdist)
+
+
 def test_cells_degenerate(sev, orc):
     """Identical points, one point far from all others, all-zero columns."""
     X = _points(5000, 12, 4, seed=3)
