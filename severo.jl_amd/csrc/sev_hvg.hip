@@ -126,7 +126,11 @@ k_loess(int64_t N, const double *x, const double *y, int64_t q, double *fit) {
 
 // standardized_var_clipped (src/variablefeatures.jl:21-28), one wavefront
 // per gene: (sum_nz min((x - mu)/sd, vmax)^2 + (m - nnz) min(-mu/sd, vmax)^2)
-// / (m - 1) for sd > 0, else 0; vmax = sqrt(m).
+// / (m - 1) for sd > 0, else 0; vmax = sqrt(m).  Lane l adds entries l, l + 64,
+// ... in order (genes with equal counts in other cells tie exactly or not by
+// this order, and ties rank by index), 8 of them loaded ahead and divided at
+// once: one load and one division at a time took 7.0 ms for the 932,747 entries
+// of the densest gene of 1M cells, now 2.0.
 __global__ void __launch_bounds__(kBlock)
 k_standardized_var(int64_t m, int64_t ncol, const int64_t *colptr, const int32_t *x,
                    const double *mu, const double *sd, double *out) {
@@ -141,10 +145,31 @@ k_standardized_var(int64_t m, int64_t ncol, const int64_t *colptr, const int32_t
     const double vmax = sqrt((double)m);
     const int64_t b = colptr[col], e = colptr[col + 1];
     double t = 0.0;
-    for (int64_t p = b + lane; p < e; p += kWave) {
-        double v = ((double)x[p] - muj) / sdj;
-        if (v > vmax) v = vmax;
-        t += v * v;
+    constexpr int U = 8;
+    int64_t p = b + lane;
+    int32_t xv[U], xn[U];
+    // positions clamped into the column: the loads stay unconditional
+    if (b < e)
+#pragma unroll
+        for (int u = 0; u < U; ++u) xv[u] = x[p + u * kWave < e ? p + u * kWave : e - 1];
+    for (; p < e; p += U * kWave) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t q = p + (U + u) * kWave;
+            xn[u] = x[q < e ? q : e - 1];
+        }
+        double w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            double v = ((double)xv[u] - muj) / sdj;
+            if (v > vmax) v = vmax;
+            w[u] = v * v;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (p + u * kWave < e) t += w[u];
+#pragma unroll
+        for (int u = 0; u < U; ++u) xv[u] = xn[u];
     }
     t = wave_sum(t);
     if (lane == 0) {

@@ -265,125 +265,134 @@ k_gather_copy(const int64_t *feat, const int64_t *colptr, const int32_t *row, co
 //   mu += delta / T(count); s += delta * (v - mu)
 // var = s / T(m - 1); sigma = sqrt(var); mu' = mu / sigma;
 // clip = scale_max + mu'.
-// Each chunk of 64 values is loaded with one coalesced read (one per lane)
-// and consumed in order through readlane; the 64 reciprocals of the chunk's
-// counts are computed in parallel by the lanes.
+// The recurrence is a serial chain, and its longest column (932,747 entries of
+// the 1M-cell variable genes) sets the time, so a step holds only the chain:
+//  - the quotient delta / T(count) by Markstein's correction step (below), five
+//    dependent operations with the addition to mu, instead of a division;
+//  - the 64 values of a chunk, their counts and the counts' reciprocals are
+//    made by the lanes in parallel and put in LDS, from where groups of 8
+//    steps take them ahead of the chain (readlane into scalar registers
+//    stalled it: 83 cycles per step in FP32, now 45; in FP64 with the division
+//    300, now 112);
+//  - whether a quotient could leave the normal range is decided per chunk, from
+//    the chunk's smallest value and mu: values and means of at least 2^-60
+//    (FP64: 2^-400) differ by zero or by 2^-84 (2^-453) or more.  Other chunks
+//    take the division itself.
+// 1M cells, the 2,000 variable genes (FP32): 32.2 -> 17.6 ms; 27,998 genes'
+// counts (FP64): 116 -> 43.5 ms.
 // --------------------------------------------------------------------------
-__device__ __forceinline__ float lane_value(float x, int t) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), t));
-}
-__device__ __forceinline__ double lane_value(double x, int t) {
-    const uint64_t u = (uint64_t)__double_as_longlong(x);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, t);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), t);
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
 
-// delta / T(count) rounded to T (the reference divides by count converted
-// to T): the FP64 form divides.
-__device__ __forceinline__ double welford_quot(double delta, double, double countf, bool) {
-    return delta / countf;
-}
-
-// The FP32 quotient RN(delta/F), F = Float32(count), by Markstein's
-// correction step (P. Markstein, IBM J. Res. Dev. 34(1), 1990): with
-// y = RN(1/F) and q = RN(delta*y) within one ulp of delta/F, r = delta - q*F
-// is exact (one fma) and RN(q + r*y) is RN(delta/F), the IEEE FP32
-// division's result.  y = RN32(RN64(1/F)) is RN32(1/F): for an
-// integer-valued F, 1/F is at least 2^-49 (relative) from every FP32
-// rounding boundary, so the second rounding cannot move it.  Every operation
-// of the recurrence's chain is FP32; deltas below 2^-90 in magnitude, whose
-// products could leave the normal range, take the exact division instead.
-__device__ __forceinline__ float welford_quot32(float delta, float F, float y) {
+// The quotient RN(delta/F), F = T(count), by Markstein's correction step
+// (P. Markstein, IBM J. Res. Dev. 34(1), 1990): with y = RN(1/F) and q =
+// RN(delta*y) within two ulps of delta/F, r = delta - q*F is exact (one fma:
+// F is an integer of at most 31 bits) and RN(q + r*y) is RN(delta/F), the IEEE
+// division's result.
+__device__ __forceinline__ float welford_quot(float delta, float F, float y) {
     const float q = delta * y;
     const float r = fmaf(-q, F, delta);
     return fmaf(r, y, q);
 }
-__device__ __forceinline__ bool welford_tiny(float delta) {
-    return fabsf(delta) < 0x1p-90f && delta != 0.0f;
+__device__ __forceinline__ double welford_quot(double delta, double F, double y) {
+    const double q = delta * y;
+    const double r = fma(-q, F, delta);
+    return fma(r, y, q);
+}
+// RN(1/F): in FP32 the rounding of the FP64 quotient (for an integer-valued F,
+// 1/F is at least 2^-49, relative, from every FP32 rounding boundary)
+__device__ __forceinline__ float welford_rcp(float F) { return (float)(1.0 / (double)F); }
+__device__ __forceinline__ double welford_rcp(double F) { return 1.0 / F; }
+template <class T>
+__device__ __forceinline__ T welford_floor() {
+    return sizeof(T) == 4 ? (T)0x1p-60 : (T)0x1p-400;
+}
+
+// A wavefront's chunk: values, counts and reciprocals of 64 steps.
+template <class T>
+struct WelfordChunk {
+    T v[kWave], F[kWave], y[kWave];
+};
+
+// mu and s of the column whose entry p < e has the value value(p), the count
+// starting at count (before the first entry).
+template <class T, class V>
+__device__ __forceinline__ void welford_column(int64_t b, int64_t e, int64_t count,
+                                               WelfordChunk<T> &L, V value, T &mu_, T &s_) {
+    const int lane = lane_id();
+    T mu = 0, s = 0;
+    // the next chunk's values are loaded while the recurrence runs over the
+    // current one (positions clamped into the column)
+    T vraw = b < e ? value(b + lane < e ? b + lane : e - 1) : T(0);
+    for (int64_t base = b; base < e; base += kWave) {
+        const T vl = vraw;
+        const int64_t pn = base + kWave + lane;
+        if (base + kWave < e) vraw = value(pn < e ? pn : e - 1);
+        const int nt = (int)((e - base) < kWave ? (e - base) : kWave);
+        const T Fl = (T)(count + lane + 1);
+        L.v[lane] = vl;
+        L.F[lane] = Fl;
+        L.y[lane] = welford_rcp(Fl);
+        const bool plain = __all(!(lane < nt) || vl >= welford_floor<T>()) &&
+                           mu >= welford_floor<T>();
+        if (plain && nt == kWave) {
+            // groups of 8 steps, the next group's operands read from LDS
+            // while the chain runs over the current ones
+            constexpr int U = 8;
+            T v[2][U], F[2][U], y[2][U];
+            auto take = [&](int g, T (&v)[U], T (&F)[U], T (&y)[U]) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) v[u] = L.v[g * U + u];
+#pragma unroll
+                for (int u = 0; u < U; ++u) F[u] = L.F[g * U + u];
+#pragma unroll
+                for (int u = 0; u < U; ++u) y[u] = L.y[g * U + u];
+            };
+            take(0, v[0], F[0], y[0]);
+#pragma unroll
+            for (int g = 0; g < kWave / U; ++g) {
+                if (g + 1 < kWave / U) take(g + 1, v[(g + 1) & 1], F[(g + 1) & 1], y[(g + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const T x = v[g & 1][u], delta = x - mu;
+                    mu = mu + welford_quot(delta, F[g & 1][u], y[g & 1][u]);
+                    s = s + delta * (x - mu);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            for (int t = 0; t < nt; ++t) {
+                const T v = L.v[t];
+                const T delta = v - mu;
+                mu = mu + delta / L.F[t];
+                s = s + delta * (v - mu);
+            }
+        }
+        count += nt;
+    }
+    mu_ = mu;
+    s_ = s;
 }
 
 template <class T>
 __global__ void __launch_bounds__(kBlock)
 k_scale_stats(int64_t m, int64_t ncol, const int64_t *colptr, const T *x, T scale_max, T *sdv,
               T *mupv, T *clipv, const int64_t *row0, int64_t S) {
+    __shared__ WelfordChunk<T> chunk[kBlock / kWave];
     const int64_t col = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
     if (col >= ncol) return;
-    const int lane = lane_id();
     if (row0) {
         // column (j, s) of a stacked batch: the rows of sample s = col % S
         const int64_t s = col % S;
         m = row0[s + 1] - row0[s];
     }
     const int64_t b = colptr[col], e = colptr[col + 1];
-    int64_t count = m - (e - b);
-    const bool fast = sizeof(T) == 4;
-    T mu = 0, s = 0;
-    // the next chunk's values are loaded while the recurrence runs over the
-    // current one (indices clamped into the column, so every load is issued
-    // and only the current chunk's is waited for; lanes past the end read 0)
-    T vraw = b < e ? x[b + lane < e ? b + lane : e - 1] : T(0);
-    for (int64_t base = b; base < e; base += kWave) {
-        const int64_t pn = base + kWave + lane;
-        const T vnext = x[pn < e ? pn : e - 1];
-        const T vl = base + lane < e ? vraw : T(0);
-        vraw = vnext;
-        // lane l: F = Float32(count + l + 1) and RN32(1/F) for element l of the chunk
-        const float fl = fast ? (float)(count + lane + 1) : 0.0f;
-        const float yl = fast ? (float)(1.0 / (double)fl) : 0.0f;
-        const int nt = (int)((e - base) < kWave ? (e - base) : kWave);
-        if constexpr (sizeof(T) == 4) {
-            // every lane holds the same mu and delta, so the rare exact
-            // division (tiny nonzero deltas) is a wave-uniform scalar branch,
-            // and full chunks run without per-element bounds checks
-            auto step = [&](int t) {
-                const float v = lane_value(vl, t);
-                const float delta = v - mu;
-                float q = welford_quot32(delta, lane_value(fl, t), lane_value(yl, t));
-                if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)welford_tiny(delta)), 0))
-                    q = delta / (float)(count + t + 1);
-                mu = mu + q;
-                s = s + delta * (v - mu);
-            };
-            if (nt == kWave) {
-                // full chunk without the per-element branch: tiny deltas are
-                // only flagged (off the recurrence chain), and a flagged
-                // chunk is redone with the exact division
-                const float mu0 = mu, s0 = s;
-                bool tiny = false;
-#pragma unroll
-                for (int t = 0; t < kWave; ++t) {
-                    const float v = lane_value(vl, t);
-                    const float delta = v - mu;
-                    tiny = tiny || welford_tiny(delta);
-                    mu = mu + welford_quot32(delta, lane_value(fl, t), lane_value(yl, t));
-                    s = s + delta * (v - mu);
-                }
-                if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)tiny), 0)) {
-                    mu = mu0;
-                    s = s0;
-                    for (int t = 0; t < kWave; ++t) step(t);
-                }
-            } else {
-                for (int t = 0; t < nt; ++t) step(t);
-            }
-        } else {
-#pragma unroll
-            for (int t = 0; t < kWave; ++t) {
-                if (t < nt) {
-                    const T v = lane_value(vl, t);
-                    const T delta = v - mu;
-                    mu = mu + welford_quot(delta, 0.0, (T)(count + t + 1), false);
-                    s = s + delta * (v - mu);
-                }
-            }
-        }
-        count += nt;
-    }
+    T mu, s;
+    welford_column<T>(b, e, m - (e - b), chunk[threadIdx.x / kWave],
+                      [&](int64_t p) { return x[p]; }, mu, s);
     const T var = s / (T)(m - 1);
     const T sd = sqrt(var);
     const T mup = mu / sd;
-    if (lane == 0) {
+    if (lane_id() == 0) {
         sdv[col] = sd;
         mupv[col] = mup;
         clipv[col] = scale_max + mup;
@@ -393,8 +402,8 @@ k_scale_stats(int64_t m, int64_t ncol, const int64_t *colptr, const T *x, T scal
 // The same statistics for many short columns (the stacked batch, column
 // (j, s) holding feature j of sample s = col % S): one lane per column, each
 // lane running its column's recurrence in the same operations and order as
-// k_scale_stats (Markstein's FP32 quotient, exact division for the tiny
-// deltas), so the results are the same bits.
+// k_scale_stats (exact division for the tiny deltas), so the results are the
+// same bits.
 __global__ void __launch_bounds__(kBlock)
 k_scale_stats_lane(int64_t ncol, const int64_t *colptr, const float *x, float scale_max,
                    float *sdv, float *mupv, float *clipv, const int64_t *row0, int64_t S) {
@@ -407,13 +416,10 @@ k_scale_stats_lane(int64_t ncol, const int64_t *colptr, const float *x, float sc
     float mu = 0.0f, s = 0.0f;
     auto step = [&](float v) {
         ++count;
-        const float F = (float)count;
+        const float F = (float)count, y = welford_rcp(F);
         const float delta = v - mu;
-        float q;
-        if (welford_tiny(delta))
-            q = delta / F;
-        else
-            q = welford_quot32(delta, F, (float)(1.0 / (double)F));
+        float q = welford_quot(delta, F, y);
+        if (fabsf(delta) < 0x1p-90f && delta != 0.0f) q = delta / F;
         mu = mu + q;
         s = s + delta * (v - mu);
     };
@@ -445,30 +451,19 @@ k_scale_stats_lane(int64_t ncol, const int64_t *colptr, const float *x, float sc
 }
 
 // mean_std(Float64, A) of the Int32 counts (src/scaling.jl:18-38,119-130):
-// the same one-wavefront-per-column Welford recurrence in FP64 (IEEE
-// division by the count), sd = sqrt(s / (m - 1)).
+// the same one-wavefront-per-column Welford recurrence in FP64, sd =
+// sqrt(s / (m - 1)).
 __global__ void __launch_bounds__(kBlock)
 k_count_mean_std(int64_t m, int64_t ncol, const int64_t *colptr, const int32_t *x, double *muv,
                  double *sdv) {
+    __shared__ WelfordChunk<double> chunk[kBlock / kWave];
     const int64_t col = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
     if (col >= ncol) return;
-    const int lane = lane_id();
     const int64_t b = colptr[col], e = colptr[col + 1];
-    int64_t count = m - (e - b);
-    double mu = 0.0, s = 0.0;
-    for (int64_t base = b; base < e; base += kWave) {
-        const int64_t p = base + lane;
-        const double vl = p < e ? (double)x[p] : 0.0;
-        const int nt = (int)((e - base) < kWave ? (e - base) : kWave);
-        for (int t = 0; t < nt; ++t) {
-            const double v = lane_value(vl, t);
-            const double delta = v - mu;
-            mu = mu + delta / (double)(count + t + 1);
-            s = s + delta * (v - mu);
-        }
-        count += nt;
-    }
-    if (lane == 0) {
+    double mu, s;
+    welford_column<double>(b, e, m - (e - b), chunk[threadIdx.x / kWave],
+                           [&](int64_t p) { return (double)x[p]; }, mu, s);
+    if (lane_id() == 0) {
         muv[col] = mu;
         sdv[col] = sqrt(s / (double)(m - 1));
     }
@@ -481,25 +476,14 @@ k_count_mean_std(int64_t m, int64_t ncol, const int64_t *colptr, const int32_t *
 __global__ void __launch_bounds__(kBlock)
 k_rel_mean_var(int64_t m, int64_t ncol, const int64_t *colptr, const int32_t *row,
                const int32_t *x, const uint32_t *tot, double *muv, double *varv) {
+    __shared__ WelfordChunk<double> chunk[kBlock / kWave];
     const int64_t col = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
     if (col >= ncol) return;
-    const int lane = lane_id();
     const int64_t b = colptr[col], e = colptr[col + 1];
-    int64_t count = m - (e - b);
-    double mu = 0.0, s = 0.0;
-    for (int64_t base = b; base < e; base += kWave) {
-        const int64_t p = base + lane;
-        const double vl = p < e ? (double)x[p] / (double)tot[row[p]] : 0.0;
-        const int nt = (int)((e - base) < kWave ? (e - base) : kWave);
-        for (int t = 0; t < nt; ++t) {
-            const double v = lane_value(vl, t);
-            const double delta = v - mu;
-            mu = mu + delta / (double)(count + t + 1);
-            s = s + delta * (v - mu);
-        }
-        count += nt;
-    }
-    if (lane == 0) {
+    double mu, s;
+    welford_column<double>(b, e, m - (e - b), chunk[threadIdx.x / kWave],
+                           [&](int64_t p) { return (double)x[p] / (double)tot[row[p]]; }, mu, s);
+    if (lane_id() == 0) {
         muv[col] = mu;
         varv[col] = s / (double)(m - 1);
     }

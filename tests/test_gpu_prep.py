@@ -203,3 +203,24 @@ def test_large_load_roundtrip_and_checks(sev):
     with pytest.raises(sev.SeveroError, match="strictly increasing"):
         p.load_counts_julia(m, n, colptr, uns, vals)
     p.close()
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 127, 129, 1000])
+def test_scale_stats_chunk_edges(sev, orc, dt, n):
+    """Columns around the recurrence's chunks of 64 entries, with values that
+    take the exact division (negative, zero, tiny) in some chunks only: sd and
+    mu' bit for bit as the oracle's sequential recurrence."""
+    rng = np.random.default_rng(n)
+    m, cols = 1500, 6
+    data = rng.lognormal(0, 1, (cols, n)).astype(dt)
+    data[1] *= dt(-1)
+    data[2, rng.random(n) < 0.05] = dt(1e-30)
+    data[3, n // 2] = dt(0)
+    data[4] = dt(3)
+    data[5, -1] = dt(-2)
+    rows = np.concatenate([np.sort(rng.choice(m, n, replace=False)) for _ in range(cols)])
+    A = sp.csc_matrix((data.ravel(), rows, np.arange(cols + 1) * n), shape=(m, cols))
+    C = sev.scale_features(A, scale_max=10.0, dtype=dt)
+    B, mu, _ = orc.scale(m, A.indptr.astype(np.int64), A.data, dt(10.0))
+    assert np.array_equal(C.A.data, B, equal_nan=True) and np.array_equal(C.mu, mu, equal_nan=True)
