@@ -442,6 +442,60 @@ k_dot_w(int64_t m, const TW *W, int jc, const double *y, double *part) {
     }
 }
 
+// The same sums with the columns dealt to the gridDim.y blocks of a slab, 4
+// each, and the 8 rows of a thread loaded together: for operators of few slabs
+// (a slab per block left 254 of 256 compute units idle at 5,000 rows: 40 us per
+// launch, now 10; 100,000 rows: 79 -> 19).  Each column is summed in the same
+// order (the butterfly's pairs are those of plain xor steps), so the bits are
+// the same.
+constexpr int kDotCols = 4;
+
+template <class TW>
+__global__ void __launch_bounds__(kDotThreads)
+k_dot_w_cols(int64_t m, const TW *W, int jc, const double *y, double *part) {
+    constexpr int NW = kDotThreads / kWave, NR = (int)(kSlabRows / kDotThreads);
+    __shared__ double red[NW][kDotCols];
+    const int64_t nblk = gridDim.x;
+    const int64_t rb = (int64_t)blockIdx.x * kSlabRows;
+    const int64_t re = rb + kSlabRows < m ? rb + kSlabRows : m;
+    const int c0 = (int)blockIdx.y * kDotCols;
+    const int w = threadIdx.x / kWave, lane = lane_id();
+    double wv[NR][kDotCols], yv[NR];
+    // every load is issued (rows and columns clamped); rows past the end are
+    // left out of the sums, columns past jc are not stored
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+        const int64_t r = rb + threadIdx.x + u * kDotThreads;
+        const int64_t rc = r < re ? r : re - 1;
+        yv[u] = y[rc];
+#pragma unroll
+        for (int i = 0; i < kDotCols; ++i)
+            wv[u][i] = (double)W[(int64_t)(c0 + i < jc ? c0 + i : jc - 1) * m + rc];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    double acc[kDotCols];
+#pragma unroll
+    for (int i = 0; i < kDotCols; ++i) acc[i] = 0.0;
+#pragma unroll
+    for (int u = 0; u < NR; ++u)
+        if (rb + threadIdx.x + u * kDotThreads < re)
+#pragma unroll
+            for (int i = 0; i < kDotCols; ++i) acc[i] = fma(wv[u][i], yv[u], acc[i]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int i = 0; i < kDotCols; ++i) acc[i] += __shfl_xor(acc[i], o, kWave);
+    if (lane == 0)
+#pragma unroll
+        for (int i = 0; i < kDotCols; ++i) red[w][i] = acc[i];
+    __syncthreads();
+    if (threadIdx.x < kDotCols && c0 + (int)threadIdx.x < jc) {
+        double u = 0.0;
+        for (int q = 0; q < NW; ++q) u += red[q][threadIdx.x];
+        part[(int64_t)(c0 + threadIdx.x) * nblk + blockIdx.x] = u;
+    }
+}
+
 // T[i] = sum_b part[i*nblk + b]: block i sums column i (each thread a
 // strided subset with independent loads, then the fixed-order block sum).
 __global__ void __launch_bounds__(kBlock) k_red_t(int nblk, const double *part, double *T) {
@@ -498,6 +552,67 @@ k_apply(int64_t m, int64_t n, const TW *W, int jc, const double *T, const double
     }
 }
 
+// y' alone, one row per thread, for operators of few slabs; the norm and the
+// sum of a slab are then taken by the A' w kernel that stages it (slab_norms,
+// the same order as k_apply's).  5,000 rows: 31 us per launch, now 8; 100,000:
+// 48, now 16.
+constexpr int kRowThreads = 128;
+
+template <class TW>
+__global__ void __launch_bounds__(kRowThreads)
+k_apply_rows(int64_t m, const TW *W, int jc, const double *T, const double *y, double *yout) {
+    __shared__ double tl[kMaxWork];
+    for (int i = threadIdx.x; i < jc; i += kRowThreads) tl[i] = T[i];
+    const int64_t r = (int64_t)blockIdx.x * kRowThreads + threadIdx.x;
+    const int64_t rc = r < m ? r : m - 1;
+    const double yv = y[rc];
+    __syncthreads();
+    double d = 0.0;
+    // 16 columns at a time: the loads first (column index clamped), then the
+    // chain in column order
+    for (int c0 = 0; c0 < jc; c0 += 16) {
+        double wv[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            wv[i] = (double)W[(int64_t)(c0 + i < jc ? c0 + i : jc - 1) * m + rc];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (c0 + i < jc) d = fma(wv[i], tl[c0 + i], d);
+    }
+    if (r < m) yout[r] = jc > 0 ? yv - d : yv;
+}
+
+// ||y'||^2 and sum(y') of a slab in k_apply's order (its thread t = tid +
+// 256 q adds rows t, t + 1024, ...; wavefronts in order), by a block of kBlock
+// threads; thread 0 stores them.
+__device__ void slab_norms(const double *y, int64_t nrows, double *out) {
+    constexpr int Q = kApplyThreads / kBlock;
+    __shared__ double sc[2][kApplyThreads / kWave];
+    const int w = threadIdx.x / kWave;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        double nrm = 0.0, sm = 0.0;
+        for (int64_t lr = threadIdx.x + q * kBlock; lr < nrows; lr += kApplyThreads) {
+            const double yv = y[lr];
+            nrm = fma(yv, yv, nrm);
+            sm += yv;
+        }
+        nrm = wave_sum(nrm);
+        sm = wave_sum(sm);
+        if (lane_id() == 0) {
+            sc[0][w + kWaves * q] = nrm;
+            sc[1][w + kWaves * q] = sm;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double s = 0.0;
+        for (int i = 0; i < kApplyThreads / kWave; ++i) s += sc[threadIdx.x][i];
+        out[threadIdx.x] = s;
+    }
+}
+
 // Workgroups are dealt to the 8 XCDs in turn (linear id mod 8).  A' w maps
 // block x to the slab that puts consecutive slabs of a column group on one
 // XCD and 8 dispatches apart: the cache lines at the boundary of a column's
@@ -532,7 +647,7 @@ __device__ __forceinline__ T group_sum(T v) {
 // arrays are padded so the cover stays in bounds); two accumulators
 // alternate and are combined in order, then the group is summed.
 // --------------------------------------------------------------------------
-template <class VT, int G>
+template <class VT, int G, bool NORMS>
 __global__ void __launch_bounds__(kBlock)
 k_atw(int64_t m, int64_t n, const int64_t *off, const uint16_t *lrow, const VT *val,
       const double *y, double *part) {
@@ -548,6 +663,8 @@ k_atw(int64_t m, int64_t n, const int64_t *off, const uint16_t *lrow, const VT *
         wl[lr] = lr < nrows ? y[r0 + lr] : 0.0;
     __syncthreads();
     double *prow = part + s * (n + 2);
+    if constexpr (NORMS)
+        if (g == 0) slab_norms(y + r0, nrows, prow + n);
     for (int64_t j0 = ((int64_t)g * kWaves + w) * C; j0 < n; j0 += (int64_t)ng * kWaves * C) {
         const int64_t j = j0 + c;
         double acc0 = 0.0, acc1 = 0.0;
@@ -599,7 +716,7 @@ __device__ __forceinline__ float atw_seg_bf16(int64_t a, int64_t b, const uint32
     return acc0 + acc1;
 }
 
-template <int G>
+template <int G, bool NORMS>
 __global__ void __launch_bounds__(kBlock)
 k_atw_bf16(int64_t m, int64_t n, const int64_t *off, const uint32_t *lrow12, const uint16_t *val,
            const double *y, double *part) {
@@ -615,6 +732,8 @@ k_atw_bf16(int64_t m, int64_t n, const int64_t *off, const uint32_t *lrow12, con
         wl[lr] = lr < nrows ? (float)y[r0 + lr] : 0.0f;
     __syncthreads();
     double *prow = part + s * (n + 2);
+    if constexpr (NORMS)
+        if (g == 0) slab_norms(y + r0, nrows, prow + n);
     for (int64_t j0 = ((int64_t)g * kWaves + w) * C; j0 < n; j0 += (int64_t)ng * kWaves * C) {
         const int64_t j = j0 + c;
         float acc = 0.0f;
@@ -1846,53 +1965,88 @@ void launch_av(const SlabCsc &op, const double *v, const double *rf, const doubl
 }
 
 int atw_groups_default(const SlabCsc &op) {
+    // 4 blocks per compute unit, each wavefront with 4 columns or more (the
+    // groups of a slab only share its columns out: no sum depends on them; at
+    // most 16 groups left 5,000 rows with 32 blocks: 43 us per launch, now 18)
     const int64_t want = ceil_div((int64_t)device_cu_count() * 4, op.nslab);
     const int64_t cap = std::max<int64_t>(1, op.n / (4 * kWaves));
-    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, 16), cap));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(want, cap));
 }
 
 int atw_groups(const SlabCsc &op) { return op.atw_groups > 0 ? op.atw_groups : atw_groups_default(op); }
 
-template <int G>
+template <int G, bool NORMS>
 void launch_atw_g(const SlabCsc &op, const double *y, double *part, hipStream_t st) {
     const dim3 grid((unsigned)op.nslab, (unsigned)atw_groups(op));
     if (op.vtype == kValBF16)
-        hipLaunchKernelGGL(k_atw_bf16<G>, grid, dim3(kBlock), 0, st, op.m, op.n, op.off.get(),
-                           op.lrow12.get(), (const uint16_t *)op.vals, y, part);
+        hipLaunchKernelGGL((k_atw_bf16<G, NORMS>), grid, dim3(kBlock), 0, st, op.m, op.n,
+                           op.off.get(), op.lrow12.get(), (const uint16_t *)op.vals, y, part);
     else if (op.vtype == kValF64)
-        hipLaunchKernelGGL((k_atw<double, G>), grid, dim3(kBlock), 0, st, op.m, op.n,
+        hipLaunchKernelGGL((k_atw<double, G, NORMS>), grid, dim3(kBlock), 0, st, op.m, op.n,
                            op.off.get(), op.lrow.get(), (const double *)op.vals, y, part);
     else
-        hipLaunchKernelGGL((k_atw<float, G>), grid, dim3(kBlock), 0, st, op.m, op.n,
+        hipLaunchKernelGGL((k_atw<float, G, NORMS>), grid, dim3(kBlock), 0, st, op.m, op.n,
                            op.off.get(), op.lrow.get(), (const float *)op.vals, y, part);
     SEV_LAUNCH_CHECK();
 }
 
-void launch_atw_only(const SlabCsc &op, const double *y, double *part, hipStream_t st) {
+void launch_atw_only(const SlabCsc &op, const double *y, double *part, hipStream_t st,
+                     bool norms = false) {
     ProfScope ps("spmv_atw", st,
                  (double)op.nnz * (val_bytes(op.vtype) + (op.vtype == kValBF16 ? 1.5 : 2.0)) +
                      8.0 * op.m + 8.0 * (op.nslab + 1) * op.n);
-    switch (op.atw_lanes) {
-        case 4: launch_atw_g<4>(op, y, part, st); break;
-        case 8: launch_atw_g<8>(op, y, part, st); break;
-        case 16: launch_atw_g<16>(op, y, part, st); break;
-        case 32: launch_atw_g<32>(op, y, part, st); break;
-        default: launch_atw_g<64>(op, y, part, st); break;
-    }
+    auto go = [&](auto nm) {
+        constexpr bool N = decltype(nm)::value;
+        switch (op.atw_lanes) {
+            case 4: launch_atw_g<4, N>(op, y, part, st); break;
+            case 8: launch_atw_g<8, N>(op, y, part, st); break;
+            case 16: launch_atw_g<16, N>(op, y, part, st); break;
+            case 32: launch_atw_g<32, N>(op, y, part, st); break;
+            default: launch_atw_g<64, N>(op, y, part, st); break;
+        }
+    };
+    if (norms)
+        go(std::true_type());
+    else
+        go(std::false_type());
 }
+
+// Fewer slabs than compute units: the reorthogonalisation kernels share each
+// slab among several blocks (from half a million rows on, one block per slab
+// fills the device, and the norms cost the A' w kernel of 1M rows 9%).
+bool few_slabs(const SlabCsc &op) { return op.nslab <= device_cu_count() / 2; }
 
 // y' = y - W[:,0:jc] T into yout (plus norm/sum partials), then the slab
 // partials of B' y'.
 template <class TW>
 void launch_upd_atw(const SlabCsc &op, const TW *W, int jc, const double *T,
                     const double *y, double *yout, double *part, hipStream_t st) {
+    const bool few = few_slabs(op);
     {
         ProfScope ps("reorth_apply", st, (double)op.m * (sizeof(TW) * jc + 16));
-        hipLaunchKernelGGL(k_apply<TW>, dim3((unsigned)op.nslab), dim3(kApplyThreads), 0, st,
-                           op.m, op.n, W, jc, T, y, yout, part);
+        if (few)
+            hipLaunchKernelGGL(k_apply_rows<TW>, dim3((unsigned)ceil_div(op.m, kRowThreads)),
+                               dim3(kRowThreads), 0, st, op.m, W, jc, T, y, yout);
+        else
+            hipLaunchKernelGGL(k_apply<TW>, dim3((unsigned)op.nslab), dim3(kApplyThreads), 0, st,
+                               op.m, op.n, W, jc, T, y, yout, part);
         SEV_LAUNCH_CHECK();
     }
-    launch_atw_only(op, yout, part, st);
+    launch_atw_only(op, yout, part, st, few);
+}
+
+// Partial dots W[:, 0:jc]' y per slab.
+template <class TW>
+void launch_dot(const SlabCsc &op, const TW *W, int jc, const double *y, double *part,
+                hipStream_t st) {
+    if (few_slabs(op))
+        hipLaunchKernelGGL(k_dot_w_cols<TW>,
+                           dim3((unsigned)op.nslab, (unsigned)((jc + kDotCols - 1) / kDotCols)),
+                           dim3(kDotThreads), 0, st, op.m, W, jc, y, part);
+    else
+        hipLaunchKernelGGL(k_dot_w<TW>, dim3((unsigned)op.nslab), dim3(kDotThreads), 0, st, op.m, W,
+                           jc, y, part);
+    SEV_LAUNCH_CHECK();
 }
 
 void launch_right_step(const SlabCsc &op, int j, int work, const double *part2, double *V,
@@ -2046,8 +2200,8 @@ void autotune_operator(SlabCsc &op, hipStream_t st) {
     // by one wavefront in the same order.
     best.lanes = op.lanes_per_row;
     const int cap = (int)std::max<int64_t>(1, op.n / (4 * kWaves));
-    for (int g : {1, 2, 3, 4, 6, 8, 12, 16}) {
-        if (g > cap) break;
+    for (int g : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+        if (g > cap || (g > 16 && !few_slabs(op))) break;
         op.atw_groups = g;
         const float ms = time_launches(st, [&] { launch_atw_only(op, y.get(), part.get(), st); }, 3);
         if (ms < best_ms) {
@@ -2207,9 +2361,7 @@ void irlba_run(const SlabCsc &op, const IrlbaParams &p, const double *init, Irlb
             const int jc = j;
             if (jc > 0) {
                 ProfScope ps("reorth_dot", st, (double)m * (sizeof(TW) * jc + 8));
-                hipLaunchKernelGGL(k_dot_w<TW>, dim3(dot_blocks), dim3(kDotThreads), 0, st, m, Wd,
-                                   jc, y, w.red.get());
-                SEV_LAUNCH_CHECK();
+                launch_dot<TW>(op, Wd, jc, y, w.red.get(), st);
                 hipLaunchKernelGGL(k_red_t, dim3(jc), dim3(kBlock), 0, st, dot_blocks,
                                    w.red.get(), w.T.get());
                 SEV_LAUNCH_CHECK();

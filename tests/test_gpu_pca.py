@@ -555,3 +555,27 @@ def test_irlba_bf16_form_layouts(sev, m, n, dens):
     Q = Ab.toarray() - mu.astype(np.float64)
     ss = np.linalg.svd(Q, compute_uv=False)
     assert np.max(np.abs(S.S - ss[:nu]) / ss[:nu]) < 1e-5
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("m", [1, 63, 4095, 4096, 4097, 8200])
+def test_few_slab_kernels_vs_oracle(sev, orc, dt, m):
+    """The reorthogonalisation kernels of operators with few slabs, at the
+    edges of a slab: a PCA of a tall matrix against numpy's SVD, and the
+    centered transposed product against the oracle (1e-13: FP64 sums)."""
+    rng = np.random.default_rng(m)
+    n = 40
+    A = sp.random(m, n, 0.4, random_state=rng, format="csc", dtype=np.float64).astype(dt)
+    mu = rng.random(n).astype(dt)
+    C = sev.CenteredMatrix(A, mu)
+    x = rng.standard_normal(m)
+    y = C.rmatvec(x)
+    D = A.toarray().astype(np.float64) - mu.astype(np.float64)
+    assert np.allclose(y, D.T @ x, rtol=1e-12, atol=1e-12 * np.sqrt(m))
+    if m < 64:
+        return
+    init = rng.standard_normal(n)
+    r = sev.irlba(C, 8, init=init, tol=1e-8, work=20)
+    s = np.linalg.svd(D, compute_uv=False)
+    assert np.max(np.abs(r.S - s[:8]) / s[:8]) < 1e-7
+    assert np.abs(r.U.T @ r.U - np.eye(8)).max() < 1e-8
