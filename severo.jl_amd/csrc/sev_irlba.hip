@@ -1286,18 +1286,6 @@ k_small_svd(int n, const double *B, double *U, double *s, double *V, int *status
     small_svd_body(n, B, U, s, V, status);
 }
 
-// The same SVD with 8 lanes per column pair (ne/2 <= 31 groups in four
-// wavefronts): columns of G and J sit in LDS with stride kSvdLd, rows n..63
-// held at zero, and lane l of a group holds rows 16k + 2l + h (k < 4, h < 2),
-// so that each of its four 16-byte LDS reads per column is one contiguous
-// 128-byte segment across the group.  Half the lanes of the 16-lane form for
-// the same rounds: the per-pair reductions and rotation formulas, repeated on
-// every lane of a group, are the bulk of a round.  For work <= kSvd8MaxWork
-// (the two arrays fit the 64 KiB of LDS a block may allocate by default).
-constexpr int kSvd8Threads = 256;
-constexpr int kSvdLd = 64;
-constexpr int kSvd8MaxWork = 62;
-
 // Sum over each group of 8 lanes (quad xor 1, quad xor 2, half-row mirror):
 // commutative steps, so the 8 lanes end with bit-identical totals.
 __device__ __forceinline__ double sum8(double v) {
@@ -1307,67 +1295,64 @@ __device__ __forceinline__ double sum8(double v) {
     return v;
 }
 
-__device__ __forceinline__ void small_svd8_body(int n, const double *B, double *U, double *s,
-                                                double *V, int *status) {
-    extern __shared__ double2 svd8_lds[];  // 16-byte aligned for the paired reads
-    const int ne = n + (n & 1);
-    double *G = (double *)svd8_lds;
-    // B itself (for U = B V diag(1/s)), or the accumulated rotations when B
-    // is too ill-conditioned for that product
-    double *J = G + ne * kSvdLd;
-    __shared__ int rotated, need_j, nsweeps;
-    __shared__ double sv[kMaxWork];
-    const int tid = threadIdx.x;
-    const int pr = tid >> 3, gl = tid & 7;
-    const int npair = ne / 2;
-    const double tol2 = kJacobiCos2;
-    if (tid == 0) {
-        need_j = 0;
-        nsweeps = 0;
+// The same SVD with 8 lanes per column pair: half the lanes of the 16-lane form
+// for the same rounds, as the per-pair reductions and rotation formulas,
+// repeated on every lane of a group, are the bulk of a round.  Columns of G = B'
+// sit in LDS in chunks of 16 rows (rows n.. held at zero); lane l of a group
+// holds rows 16k + 2l + h (h < 2), so that each of its 16-byte accesses is one
+// contiguous 128-byte chunk across the group.  With SWZ = 1 chunk k of column c
+// is stored as chunk k ^ (c & 1): neighbouring groups work on neighbouring
+// columns, whose chunks then fall into different halves of the 64 banks.  It pays
+// where the rounds are bound by LDS (112 columns: a call of 1.57 ms became 1.31,
+// against columns padded by 16 bytes), not where they are one chain of latencies
+// (57 columns: 880 cycles per round, 920 with it).
+template <int KC, int LD, int SWZ>
+struct SvdCols {
+    static_assert(KC * 16 <= LD && KC % 2 == 0, "column stride");
+    // row i of column c
+    static __device__ __forceinline__ int at(int c, int i) {
+        return c * LD + ((((i >> 4) ^ (c & SWZ)) << 4) | (i & 15));
     }
-    auto load = [&](bool withj) {
-        for (int e = tid; e < ne * kSvdLd; e += kSvd8Threads) {
-            const int c = e / kSvdLd, i = e % kSvdLd;
-            const bool in = c < n && i < n;
-            G[e] = in ? B[(int64_t)i * n + c] : 0.0;  // G(i, c) = B(c, i)
-            J[e] = withj ? (in && i == c ? 1.0 : 0.0) : (in ? B[(int64_t)c * n + i] : 0.0);
-        }
-        __syncthreads();
-    };
-    auto sweeps = [&](bool withj) {
+    // lane gl's pair of chunk k
+    static __device__ __forceinline__ double2 *pair(double *G, int c, int k, int gl) {
+        return (double2 *)(G + c * LD + 16 * (k ^ (c & SWZ))) + gl;
+    }
+    // Sweeps until one rotates nothing (100 at most).  Called by all threads
+    // after a barrier; ends with one.
+    template <bool WITHJ>
+    static __device__ __forceinline__ void sweeps(int n, double *G, double *J, int *rotated,
+                                                  int *nsweeps) {
+        const int tid = threadIdx.x;
+        const int ne = n + (n & 1), N = ne - 1;
+        const int pr = tid >> 3, gl = tid & 7;
         for (int sweep = 0; sweep < 100; ++sweep) {
-            if (tid == 0) rotated = 0;
+            if (tid == 0) *rotated = 0;
             __syncthreads();
-            // circle schedule: round r pairs (r + pr, r - pr) mod (ne - 1),
-            // group 0 pairs r with the fixed column ne - 1
-            int pp = pr, qq = ne - 1 - pr;
-            for (int r = 0; r < ne - 1; ++r) {
-                if (pr < npair) {
+            int pp = pr, qq = N - pr;
+            for (int r = 0; r < N; ++r) {
+                if (pr < ne / 2) {
                     const int p = pp < qq ? pp : qq, q = pp < qq ? qq : pp;
-                    const bool valid = q < n;
-                    double2 *gp = (double2 *)(G + p * kSvdLd) + gl;
-                    double2 *gq = (double2 *)(G + q * kSvdLd) + gl;
-                    double2 x[4], y[4];
+                    double2 x[KC], y[KC];
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        x[k] = gp[8 * k];
-                        y[k] = gq[8 * k];
+                    for (int e = 0; e < KC; ++e) {
+                        x[e] = *pair(G, p, e, gl);
+                        y[e] = *pair(G, q, e, gl);
                     }
                     double app = 0.0, aqq = 0.0, apq = 0.0;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        app = fma(x[k].x, x[k].x, app);
-                        aqq = fma(y[k].x, y[k].x, aqq);
-                        apq = fma(x[k].x, y[k].x, apq);
-                        app = fma(x[k].y, x[k].y, app);
-                        aqq = fma(y[k].y, y[k].y, aqq);
-                        apq = fma(x[k].y, y[k].y, apq);
+                    for (int e = 0; e < KC; ++e) {
+                        app = fma(x[e].x, x[e].x, app);
+                        aqq = fma(y[e].x, y[e].x, aqq);
+                        apq = fma(x[e].x, y[e].x, apq);
+                        app = fma(x[e].y, x[e].y, app);
+                        aqq = fma(y[e].y, y[e].y, aqq);
+                        apq = fma(x[e].y, y[e].y, apq);
                     }
                     app = sum8(app);
                     aqq = sum8(aqq);
                     apq = sum8(apq);
-                    if (valid && apq != 0.0 && apq * apq > tol2 * app * aqq) {
-                        if (gl == 0) rotated = 1;
+                    if (q < n && apq != 0.0 && apq * apq > kJacobiCos2 * app * aqq) {
+                        if (gl == 0) *rotated = 1;
                         // t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)), c = 1/sqrt(1 + t^2)
                         const double zeta = (aqq - app) * rcp_nr(2.0 * apq);
                         const double az = fabs(zeta);
@@ -1381,42 +1366,104 @@ __device__ __forceinline__ void small_svd8_body(int n, const double *B, double *
                         const double c = rsq_nr(fma(t, t, 1.0));
                         const double sn = c * t;
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) {
-                            gp[8 * k] = make_double2(c * x[k].x - sn * y[k].x, c * x[k].y - sn * y[k].y);
-                            gq[8 * k] = make_double2(sn * x[k].x + c * y[k].x, sn * x[k].y + c * y[k].y);
+                        for (int e = 0; e < KC; ++e) {
+                            *pair(G, p, e, gl) = make_double2(c * x[e].x - sn * y[e].x,
+                                                              c * x[e].y - sn * y[e].y);
+                            *pair(G, q, e, gl) = make_double2(sn * x[e].x + c * y[e].x,
+                                                              sn * x[e].y + c * y[e].y);
                         }
-                        if (withj) {
-                            double2 *jp = (double2 *)(J + p * kSvdLd) + gl;
-                            double2 *jq = (double2 *)(J + q * kSvdLd) + gl;
+                        if (WITHJ) {
 #pragma unroll
-                            for (int k = 0; k < 4; ++k) {
-                                const double2 u = jp[8 * k], v = jq[8 * k];
-                                jp[8 * k] = make_double2(c * u.x - sn * v.x, c * u.y - sn * v.y);
-                                jq[8 * k] = make_double2(sn * u.x + c * v.x, sn * u.y + c * v.y);
+                            for (int e = 0; e < KC; ++e) {
+                                double2 *jp = pair(J, p, e, gl), *jq = pair(J, q, e, gl);
+                                const double2 u = *jp, v = *jq;
+                                *jp = make_double2(c * u.x - sn * v.x, c * u.y - sn * v.y);
+                                *jq = make_double2(sn * u.x + c * v.x, sn * u.y + c * v.y);
                             }
                         }
                     }
                 }
                 __syncthreads();
-                pp = pp + 1 == ne - 1 ? 0 : pp + 1;
-                if (pr > 0) qq = qq + 1 == ne - 1 ? 0 : qq + 1;
+                pp = pp + 1 == N ? 0 : pp + 1;
+                if (pr > 0) qq = qq + 1 == N ? 0 : qq + 1;
             }
-            const int any = rotated;
+            const int any = *rotated;
             __syncthreads();
-            if (tid == 0) nsweeps = nsweeps + 1;
+            if (tid == 0) *nsweeps = *nsweeps + 1;
             if (!any) break;
         }
+        __syncthreads();
+    }
+};
+
+// Ranks of the singular values by descending value, ties by column, and s in
+// that order; status[0] = 1 if one vanished.  One ballot per column and 64
+// values.  Called by all threads; ends with a barrier.
+__device__ __forceinline__ void svd_ranks(int n, const double *sv, int *rank, double *s,
+                                          int *status) {
+    const int l = threadIdx.x & 63;
+    for (int j = threadIdx.x >> 6; j < n; j += blockDim.x >> 6) {
+        const double sj = sv[j];
+        int rk = 0;
+        for (int i0 = 0; i0 < n; i0 += 64) {
+            const int i = i0 + l;
+            const double si = i < n ? sv[i] : 0.0;
+            rk += __popcll(__ballot(i < n && (si > sj || (si == sj && i < j))));
+        }
+        if (l == 0) {
+            rank[j] = rk;
+            s[rk] = sj;
+            if (!(sj > 0.0)) status[0] = 1;
+        }
+    }
+    __syncthreads();
+}
+
+// For work <= kSvd8MaxWork: at most 31 groups in four wavefronts, G and a
+// second array in LDS (the 64 KiB a block may allocate by default).
+constexpr int kSvd8Threads = 256;
+constexpr int kSvdLd = 64;
+constexpr int kSvd8MaxWork = 62;
+using Svd8Cols = SvdCols<4, kSvdLd, 0>;
+
+__device__ __forceinline__ void small_svd8_body(int n, const double *B, double *U, double *s,
+                                                double *V, int *status) {
+    extern __shared__ double2 svd8_lds[];  // 16-byte aligned for the paired reads
+    const int ne = n + (n & 1);
+    double *G = (double *)svd8_lds;
+    // B itself (for U = B V diag(1/s)), or the accumulated rotations when B
+    // is too ill-conditioned for that product
+    double *J = G + ne * kSvdLd;
+    __shared__ int rotated, need_j, nsweeps;
+    __shared__ double sv[kMaxWork];
+    __shared__ int rank[kMaxWork];
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        need_j = 0;
+        nsweeps = 0;
+    }
+    auto load = [&](bool withj) {
+        for (int e = tid; e < ne * kSvdLd; e += kSvd8Threads) {
+            const int c = e / kSvdLd, i = e % kSvdLd, o = Svd8Cols::at(c, i);
+            const bool in = c < n && i < n;
+            G[o] = in ? B[(int64_t)i * n + c] : 0.0;  // G(i, c) = B(c, i)
+            J[o] = withj ? (in && i == c ? 1.0 : 0.0) : (in ? B[(int64_t)c * n + i] : 0.0);
+        }
+        __syncthreads();
     };
     auto norms = [&]() {
         if (tid < n) {
             double t = 0.0;
-            for (int i = 0; i < n; ++i) t += G[tid * kSvdLd + i] * G[tid * kSvdLd + i];
+            for (int i = 0; i < n; ++i) {
+                const double x = G[Svd8Cols::at(tid, i)];
+                t += x * x;
+            }
             sv[tid] = sqrt(t);
         }
         __syncthreads();
     };
     load(false);
-    sweeps(false);
+    Svd8Cols::sweeps<false>(n, G, J, &rotated, &nsweeps);
     norms();
     // U = B V diag(1/s) is accurate to eps s_max / s_j: without the
     // accumulated rotations only while s_min >= 1e-5 s_max
@@ -1432,7 +1479,7 @@ __device__ __forceinline__ void small_svd8_body(int n, const double *B, double *
     const bool withj = need_j != 0;
     if (withj) {
         load(true);
-        sweeps(true);
+        Svd8Cols::sweeps<true>(n, G, J, &rotated, &nsweeps);
         norms();
     }
     if (tid == 0) {
@@ -1440,25 +1487,47 @@ __device__ __forceinline__ void small_svd8_body(int n, const double *B, double *
         status[1] = nsweeps;
     }
     __syncthreads();
-    for (int j = tid >> 6; j < n; j += kSvd8Threads / 64) {
-        const int l = tid & 63;
-        const double sj = sv[j];
-        int rk = 0;
-        for (int i = 0; i < n; ++i) rk += (sv[i] > sj || (sv[i] == sj && i < j)) ? 1 : 0;
-        if (l == 0) {
-            s[rk] = sj;
-            if (!(sj > 0.0)) status[0] = 1;
-        }
-        for (int i = l; i < n; i += 64) {
-            if (withj) {
-                U[(int64_t)rk * n + i] = J[j * kSvdLd + i];
-            } else {
-                // (B g_j)_i / s_j^2, g_j = s_j v_j the column of G
-                double t = 0.0;
-                for (int c = 0; c < n; ++c) t = fma(J[c * kSvdLd + i], G[j * kSvdLd + c], t);
-                U[(int64_t)rk * n + i] = t / (sj * sj);
+    svd_ranks(n, sv, rank, s, status);
+    // U = B G diag(1/s^2) and V = G diag(1/s), 4 rows x 4 columns per thread: the
+    // sums run over c in order, 16 of them side by side (one sum per lane at a
+    // time, and ranks counted entry by entry, took 60 of 170 us at 57 columns)
+    const int i0 = 4 * (tid & 15), j0 = 4 * (tid >> 4);
+    if (i0 >= n || j0 >= n) return;
+    double t[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[q][e] = 0.0;
+    if (!withj)
+        for (int c0 = 0; c0 < n; c0 += 2) {
+            // column ne - 1 and row n of G are zero or present: n even or odd
+            const double2 *b0 = (const double2 *)(J + c0 * kSvdLd + i0);
+            const double2 *b1 = (const double2 *)(J + (c0 + 1) * kSvdLd + i0);
+            const double2 p0 = b0[0], p1 = b0[1], r0 = b1[0], r1 = b1[1];
+            const double u0[4] = {p0.x, p0.y, p1.x, p1.y}, u1[4] = {r0.x, r0.y, r1.x, r1.y};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int j = j0 + q < n ? j0 + q : j0;
+                const double2 g = *(const double2 *)(G + j * kSvdLd + c0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    t[q][e] = fma(u0[e], g.x, t[q][e]);
+                    if (c0 + 1 < n) t[q][e] = fma(u1[e], g.y, t[q][e]);
+                }
             }
-            V[(int64_t)rk * n + i] = sj > 0.0 ? G[j * kSvdLd + i] / sj : 0.0;
+        }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int j = j0 + q;
+        if (j >= n) break;
+        const double sj = sv[j];
+        const int64_t o = (int64_t)rank[j] * n;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = i0 + e;
+            if (i >= n) break;
+            U[o + i] = withj ? J[j * kSvdLd + i] : t[q][e] / (sj * sj);
+            V[o + i] = sj > 0.0 ? G[j * kSvdLd + i] / sj : 0.0;
         }
     }
 }
@@ -1468,103 +1537,40 @@ k_small_svd8(int n, const double *B, double *U, double *s, double *V, int *statu
     small_svd8_body(n, B, U, s, V, status);
 }
 
-// The same SVD for 64 < work <= kMaxWork with 8 lanes per column pair (64
-// groups in eight wavefronts, circle schedule): lane l of a group holds rows
-// 16k + 2l + h (k < 8, h < 2) of its two columns, read and written as
-// 16-byte pairs; only G = B' sits in LDS (columns of kSvdLdB doubles, rows
-// n.. held at zero), so U = B V diag(1/s) reads B from global memory.  When
-// B is too ill-conditioned for that product (s_min < 1e-5 s_max) the kernel
-// sets status[0] and the caller redoes the SVD on the host (the accumulated
-// rotations would need a second n x n array).  Per round the per-pair
-// reductions and rotation formulas, repeated on every lane of a group, are
-// half those of 16 lanes per pair.
+// For 64 < work <= kMaxWork: up to 64 groups in eight wavefronts; only G sits
+// in LDS, so U = B V diag(1/s) reads B from global memory.  When B is too
+// ill-conditioned for that product (s_min < 1e-5 s_max) the kernel sets
+// status[0] and the caller redoes the SVD on the host (the accumulated
+// rotations would need a second n x n array).
 constexpr int kSvdBigThreads = 512;
-constexpr int kSvdLdB = 130;  // column stride (doubles): 128 rows + 16 bytes
+constexpr int kSvdLdB = 128;  // column stride (doubles)
+using SvdBigCols = SvdCols<8, kSvdLdB, 1>;
 
 __global__ void __launch_bounds__(kSvdBigThreads)
 k_small_svd_big(int n, const double *B, double *U, double *s, double *V, int *status) {
     extern __shared__ double2 svdb_lds[];
-    double *G = (double *)svdb_lds;  // G(i, c) = B(c, i) at G[c * kSvdLdB + i]
+    double *G = (double *)svdb_lds;  // G(i, c) = B(c, i) at G[SvdBigCols::at(c, i)]
     __shared__ int rotated, nsweeps, ill;
     __shared__ double sv[kMaxWork];
+    __shared__ int rank[kMaxWork];
     const int tid = threadIdx.x;
     const int ne = n + (n & 1);
-    const int npair = ne / 2;
-    const int pr = tid >> 3, gl = tid & 7;
-    const double tol2 = kJacobiCos2;
     if (tid == 0) {
         nsweeps = 0;
         ill = 0;
     }
     for (int e = tid; e < ne * kSvdLdB; e += kSvdBigThreads) {
         const int c = e / kSvdLdB, i = e % kSvdLdB;
-        G[e] = (c < n && i < n) ? B[(int64_t)i * n + c] : 0.0;
+        G[SvdBigCols::at(c, i)] = (c < n && i < n) ? B[(int64_t)i * n + c] : 0.0;
     }
     __syncthreads();
-    for (int sweep = 0; sweep < 100; ++sweep) {
-        if (tid == 0) rotated = 0;
-        __syncthreads();
-        // circle schedule: round r pairs (r + pr, r - pr) mod (ne - 1), group
-        // 0 pairs r with the fixed column ne - 1
-        int pp = pr, qq = ne - 1 - pr;
-        for (int r = 0; r < ne - 1; ++r) {
-            if (pr < npair) {
-                const int p = pp < qq ? pp : qq, q = pp < qq ? qq : pp;
-                const bool valid = q < n;
-                double2 *gp = (double2 *)(G + p * kSvdLdB) + gl;
-                double2 *gq = (double2 *)(G + q * kSvdLdB) + gl;
-                double2 x[8], y[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    x[k] = gp[8 * k];
-                    y[k] = gq[8 * k];
-                }
-                double app = 0.0, aqq = 0.0, apq = 0.0;
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    app = fma(x[k].x, x[k].x, app);
-                    aqq = fma(y[k].x, y[k].x, aqq);
-                    apq = fma(x[k].x, y[k].x, apq);
-                    app = fma(x[k].y, x[k].y, app);
-                    aqq = fma(y[k].y, y[k].y, aqq);
-                    apq = fma(x[k].y, y[k].y, apq);
-                }
-                app = sum8(app);
-                aqq = sum8(aqq);
-                apq = sum8(apq);
-                if (valid && apq != 0.0 && apq * apq > tol2 * app * aqq) {
-                    if (gl == 0) rotated = 1;
-                    // t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)), c = 1/sqrt(1 + t^2)
-                    const double zeta = (aqq - app) * rcp_nr(2.0 * apq);
-                    const double az = fabs(zeta);
-                    double t;
-                    if (az > 1e150) {
-                        t = 0.5 * rcp_nr(zeta);
-                    } else {
-                        const double xx = fma(az, az, 1.0);
-                        t = copysign(rcp_nr(az + xx * rsq_nr(xx)), zeta);
-                    }
-                    const double c = rsq_nr(fma(t, t, 1.0));
-                    const double sn = c * t;
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        gp[8 * k] = make_double2(c * x[k].x - sn * y[k].x, c * x[k].y - sn * y[k].y);
-                        gq[8 * k] = make_double2(sn * x[k].x + c * y[k].x, sn * x[k].y + c * y[k].y);
-                    }
-                }
-            }
-            __syncthreads();
-            pp = pp + 1 == ne - 1 ? 0 : pp + 1;
-            if (pr > 0) qq = qq + 1 == ne - 1 ? 0 : qq + 1;
-        }
-        const int any = rotated;
-        __syncthreads();
-        if (tid == 0) nsweeps = nsweeps + 1;
-        if (!any) break;
-    }
+    SvdBigCols::sweeps<false>(n, G, nullptr, &rotated, &nsweeps);
     if (tid < n) {
         double t = 0.0;
-        for (int i = 0; i < n; ++i) t += G[tid * kSvdLdB + i] * G[tid * kSvdLdB + i];
+        for (int i = 0; i < n; ++i) {
+            const double x = G[SvdBigCols::at(tid, i)];
+            t += x * x;
+        }
         sv[tid] = sqrt(t);
     }
     __syncthreads();
@@ -1584,6 +1590,7 @@ k_small_svd_big(int n, const double *B, double *U, double *s, double *V, int *st
     // columns j = w + 8q of wavefront w: lane l holds rows l and l + 64 of B,
     // loaded in blocks of 16 columns with every load in flight, and applies
     // each block to all the wavefront's j (the sums run over c in order)
+    svd_ranks(n, sv, rank, s, status);
     constexpr int kJw = kMaxWork / (kSvdBigThreads / 64);
     const int w = tid >> 6, l = tid & 63;
     for (int ih = 0; ih * 64 < n; ++ih) {
@@ -1601,9 +1608,13 @@ k_small_svd_big(int n, const double *B, double *U, double *s, double *V, int *st
                 const int j = w + 8 * q;
                 if (j < n) {
                     // rows n.. of G are zero
+                    const double2 *gj = (const double2 *)(G + SvdBigCols::at(j, c0));
 #pragma unroll
-                    for (int u = 0; u < 16; ++u)
-                        acc[q] = fma(bv[u], G[j * kSvdLdB + c0 + u], acc[q]);
+                    for (int u = 0; u < 8; ++u) {
+                        const double2 g = gj[u];
+                        acc[q] = fma(bv[2 * u], g.x, acc[q]);
+                        acc[q] = fma(bv[2 * u + 1], g.y, acc[q]);
+                    }
                 }
             }
         }
@@ -1612,12 +1623,10 @@ k_small_svd_big(int n, const double *B, double *U, double *s, double *V, int *st
             const int j = w + 8 * q;
             if (j >= n) break;
             const double sj = sv[j];
-            int rk = 0;
-            for (int r = 0; r < n; ++r) rk += (sv[r] > sj || (sv[r] == sj && r < j)) ? 1 : 0;
-            if (ih == 0 && l == 0) s[rk] = sj;
+            const int rk = rank[j];
             if (i < n) {
                 U[(int64_t)rk * n + i] = acc[q] / (sj * sj);
-                V[(int64_t)rk * n + i] = G[j * kSvdLdB + i] / sj;
+                V[(int64_t)rk * n + i] = G[SvdBigCols::at(j, i)] / sj;
             }
         }
     }

@@ -579,3 +579,24 @@ def test_few_slab_kernels_vs_oracle(sev, orc, dt, m):
     s = np.linalg.svd(D, compute_uv=False)
     assert np.max(np.abs(r.S - s[:8]) / s[:8]) < 1e-7
     assert np.abs(r.U.T @ r.U - np.eye(8)).max() < 1e-8
+
+
+@pytest.mark.parametrize("fall", [0.0, 0.12])
+@pytest.mark.parametrize("work", [12, 13, 61, 62, 63, 64, 65, 127, 128])
+def test_projected_svd_sizes_vs_oracle(sev, orc, work, fall):
+    """The projected SVD at the edges of its kernels (62, 64 and 128 Lanczos
+    vectors, odd and even), of a matrix with a flat spectrum and of one whose
+    projection falls below 1e-5 of its largest value (accumulated rotations, or
+    the host's SVD): values, residuals and orthogonality against numpy's."""
+    rng = np.random.default_rng(work)
+    m, n, nu = 400, 160, 6
+    D = rng.standard_normal((m, n)) * 10.0 ** (-fall * np.arange(n))
+    A = sp.csc_matrix(D)
+    C = sev.CenteredMatrix(A, np.zeros(n))
+    r = sev.irlba(C, nu, init=rng.standard_normal(n), tol=1e-9, work=work, maxit=2000)
+    s = np.linalg.svd(D, compute_uv=False)
+    assert np.max(np.abs(r.S - s[:nu]) / s[:nu]) < 1e-9
+    assert np.abs(r.U.T @ r.U - np.eye(nu)).max() < 1e-9
+    assert np.abs(r.V.T @ r.V - np.eye(nu)).max() < 1e-9
+    # A V = U S to the stopping tolerance
+    assert np.abs(D @ r.V - r.U * r.S).max() < 1e-8 * s[0]
