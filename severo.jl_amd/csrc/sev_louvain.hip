@@ -141,37 +141,18 @@ struct MoveRule {
     }
 };
 
-// One wave per node of at most kCap / 2 edges: all nodes (list == nullptr;
-// nodes with more edges are left to the listed launches) or the nodes of a
-// list.
+// The move of one node of at most kCap / 2 edges by a wavefront: its edges hash
+// into a table of the wavefront in LDS.  The lane's first edge (target a0,
+// weight w0, lane < deg) is loaded by the caller.
 template <int kCap>
-__global__ void __launch_bounds__(kLvThreads)
-k_move_light(int64_t n, const int32_t *list, const int64_t *ptr, const int32_t *adj,
-             const u64 *w, const u64 *k, const int32_t *c, const u64 *wtot, int32_t *cnew,
-             double totw, double res, uint64_t akey, uint32_t athresh, int *moved) {
-    __shared__ int skey[kLvWaves][kCap];
-    __shared__ u64 sval[kLvWaves][kCap];
-    const int lane = lane_id(), wv = (int)(threadIdx.x >> 6);
-    const int64_t t = (int64_t)blockIdx.x * kLvWaves + wv;
-    if (t >= n) return;
-    const int64_t v = list ? (int64_t)list[t] : t;
-    const int64_t p0 = ptr[v];
-    const int64_t deg = ptr[v + 1] - p0;
-    if (deg > kCap / 2) return;
-    const int cv = c[v];
-    if (deg == 0 || !active(v, akey, athresh)) {
-        if (lane == 0) cnew[v] = cv;
-        return;
-    }
-    // each lane's first edge is gathered while the table is cleared
+__device__ __forceinline__ int move_node(int64_t p0, int deg, int cv, u64 kvi, u64 wcv, int a0,
+                                         u64 w0, const int32_t *adj, const u64 *w,
+                                         const int32_t *c, const u64 *wtot, double totw,
+                                         double res, int *keys, u64 *vals) {
+    const int lane = lane_id();
+    // each lane's first label is gathered while the table is cleared
     int c0 = -1;
-    u64 w0 = 0;
-    if (lane < deg) {
-        c0 = c[adj[p0 + lane]];
-        w0 = w[p0 + lane];
-    }
-    int *keys = skey[wv];
-    u64 *vals = sval[wv];
+    if (lane < deg) c0 = c[a0];
     // table of the smallest power of two >= 2 deg, at least one slot a lane
     uint32_t cap = kWave;
     int shift = 26;
@@ -186,11 +167,10 @@ k_move_light(int64_t n, const int32_t *list, const int64_t *ptr, const int32_t *
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     __builtin_amdgcn_wave_barrier();
     if (lane < deg) hash_add_pow2(keys, vals, cap, shift, c0, w0);
-    for (int64_t e = lane + kWave; e < deg; e += kWave)
+    for (int e = lane + kWave; e < deg; e += kWave)
         hash_add_pow2(keys, vals, cap, shift, c[adj[p0 + e]], w[p0 + e]);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     __builtin_amdgcn_wave_barrier();
-    const u64 kvi = k[v];
     const MoveRule r{cv, res * (double)kvi / totw};
     double bs = -INFINITY;
     int bc = INT_MAX;
@@ -201,22 +181,79 @@ k_move_light(int64_t n, const int32_t *list, const int64_t *ptr, const int32_t *
     }
     wave_best(bs, bc);
     kcv = wave_max_u64(kcv);
-    if (lane == 0) {
-        const int to = r.decide(bs, bc, kcv, wtot[cv], kvi);
-        cnew[v] = to;
-        if (to != cv) atomicAdd(moved, 1);
-    }
+    __builtin_amdgcn_wave_barrier();  // the table is cleared next
+    return r.decide(bs, bc, kcv, wcv, kvi);
 }
 
-// Nodes with more than kLightDeg edges: one block each, hashing into a
-// global table of 2 * deg slots at offset 2 * ptr[v].
+// The move of node v by a wavefront, or its label if it may not move.
+template <int kCap>
+__device__ __forceinline__ void move_wave(int64_t v, int64_t p0, int deg, const int32_t *adj,
+                                          const u64 *w, const u64 *k, const int32_t *c,
+                                          const u64 *wtot, int32_t *cnew, double totw, double res,
+                                          uint64_t akey, uint32_t athresh, int *keys, u64 *vals) {
+    const int lane = lane_id();
+    const int cv = c[v];
+    int to = cv;
+    if (deg > 0 && active(v, akey, athresh)) {
+        const int a0 = lane < deg ? adj[p0 + lane] : 0;
+        const u64 w0 = lane < deg ? w[p0 + lane] : 0;
+        to = move_node<kCap>(p0, deg, cv, k[v], wtot[cv], a0, w0, adj, w, c, wtot, totw, res, keys,
+                             vals);
+    }
+    if (lane == 0) cnew[v] = to;
+}
+
+// All nodes of at most kSmallDeg edges, one per wavefront (the others are left to
+// the launch below).  Several nodes per wavefront, their scalars loaded at once
+// and the next node's edges ahead, are slower: 50,000 nodes cluster in 94, 96 and
+// 100 ms with 2, 4 and 8, in 92 with one.  The sweep's flag is not kept here: a
+// counter of the moves, or a flag stored by each, serialises them (28 and 60 us
+// a sweep).
 __global__ void __launch_bounds__(kLvThreads)
-k_move_heavy(const int32_t *heavy, const int64_t *ptr, const int32_t *adj, const u64 *w,
-             const u64 *k, const int32_t *c, const u64 *wtot, int32_t *cnew, int *hkeys,
-             u64 *hvals, double totw, double res, uint64_t akey, uint32_t athresh, int *moved) {
+k_move_light(int64_t n, const int64_t *ptr, const int32_t *adj, const u64 *w, const u64 *k,
+             const int32_t *c, const u64 *wtot, int32_t *cnew, double totw, double res,
+             uint64_t akey, uint32_t athresh) {
+    __shared__ int skey[kLvWaves][2 * kSmallDeg];
+    __shared__ u64 sval[kLvWaves][2 * kSmallDeg];
+    const int wv = (int)(threadIdx.x >> 6);
+    const int64_t v = (int64_t)blockIdx.x * kLvWaves + wv;
+    if (v >= n) return;
+    const int64_t p0 = ptr[v], deg = ptr[v + 1] - p0;
+    if (deg > kSmallDeg) return;
+    move_wave<2 * kSmallDeg>(v, p0, (int)deg, adj, w, k, c, wtot, cnew, totw, res, akey, athresh,
+                             skey[wv], sval[wv]);
+}
+
+// The nodes of more than kSmallDeg edges in one launch.  Blocks [0, nheavy): a node
+// of more than kLightDeg edges each, hashing into LDS up to kBlockDeg edges, beyond
+// into a global table of 2 * deg slots at offset 2 * ptr[v].  The others: a medium
+// node per wavefront.  Reduced networks have few of either, so that two launches
+// are two chains of latencies one after the other (15 + 17 us a sweep at 50,000
+// nodes with global tables; one launch with LDS tables 10).
+constexpr int kBlockDeg = 1024;
+constexpr int kBlockCap = 2 * kBlockDeg;
+static_assert(kBlockCap >= kLvWaves * 2 * kLightDeg, "the medium nodes' tables");
+__global__ void __launch_bounds__(kLvThreads)
+k_move_large(const int32_t *heavy, int nheavy, const int32_t *medium, int64_t nmedium,
+             const int64_t *ptr, const int32_t *adj, const u64 *w, const u64 *k, const int32_t *c,
+             const u64 *wtot, int32_t *cnew, int *hkeys, u64 *hvals, double totw, double res,
+             uint64_t akey, uint32_t athresh) {
+    __shared__ int lkeys[kBlockCap];
+    __shared__ u64 lvals[kBlockCap];
     __shared__ double rs[kLvWaves];
     __shared__ int rc[kLvWaves];
     __shared__ u64 rk[kLvWaves];
+    const int lane = lane_id(), wv = (int)(threadIdx.x >> 6);
+    if ((int)blockIdx.x >= nheavy) {
+        const int64_t t = ((int64_t)blockIdx.x - nheavy) * kLvWaves + wv;
+        if (t >= nmedium) return;
+        const int64_t v = medium[t];
+        const int64_t p0 = ptr[v];
+        move_wave<2 * kLightDeg>(v, p0, (int)(ptr[v + 1] - p0), adj, w, k, c, wtot, cnew, totw,
+                                 res, akey, athresh, lkeys + 2 * kLightDeg * wv,
+                                 lvals + 2 * kLightDeg * wv);
+        return;
+    }
     const int64_t v = heavy[blockIdx.x];
     if (!active(v, akey, athresh)) {
         if (threadIdx.x == 0) cnew[v] = c[v];
@@ -224,35 +261,51 @@ k_move_heavy(const int32_t *heavy, const int64_t *ptr, const int32_t *adj, const
     }
     const int64_t p0 = ptr[v];
     const int64_t deg = ptr[v + 1] - p0;
-    const uint32_t cap = (uint32_t)(2 * deg);
-    int *keys = hkeys + 2 * p0;
-    u64 *vals = hvals + 2 * p0;
-    for (uint32_t s = threadIdx.x; s < cap; s += kLvThreads) {
-        keys[s] = -1;
-        vals[s] = 0;
-    }
-    __threadfence();
-    __syncthreads();
-    for (int64_t e = threadIdx.x; e < deg; e += kLvThreads)
-        hash_add(keys, vals, cap, c[adj[p0 + e]], w[p0 + e]);
-    __threadfence();
-    __syncthreads();
     const int cv = c[v];
     const u64 kvi = k[v];
     const MoveRule r{cv, res * (double)kvi / totw};
     double bs = -INFINITY;
     int bc = INT_MAX;
     u64 kcv = 0;
-    for (uint32_t s = threadIdx.x; s < cap; s += kLvThreads) {
-        const int C = __hip_atomic_load(&keys[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (C >= 0)
-            r.consider(C, __hip_atomic_load(&vals[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                       wtot, bs, bc, kcv);
+    if (deg <= kBlockDeg) {
+        for (int s = threadIdx.x; s < kBlockCap; s += kLvThreads) {
+            lkeys[s] = -1;
+            lvals[s] = 0;
+        }
+        __syncthreads();
+        for (int64_t e = threadIdx.x; e < deg; e += kLvThreads)
+            hash_add_pow2(lkeys, lvals, kBlockCap, 32 - __builtin_ctz(kBlockCap), c[adj[p0 + e]],
+                          w[p0 + e]);
+        __syncthreads();
+        for (int s = threadIdx.x; s < kBlockCap; s += kLvThreads) {
+            const int C = lkeys[s];
+            if (C >= 0) r.consider(C, lvals[s], wtot, bs, bc, kcv);
+        }
+    } else {
+        const uint32_t cap = (uint32_t)(2 * deg);
+        int *keys = hkeys + 2 * p0;
+        u64 *vals = hvals + 2 * p0;
+        for (uint32_t s = threadIdx.x; s < cap; s += kLvThreads) {
+            keys[s] = -1;
+            vals[s] = 0;
+        }
+        __threadfence();
+        __syncthreads();
+        for (int64_t e = threadIdx.x; e < deg; e += kLvThreads)
+            hash_add(keys, vals, cap, c[adj[p0 + e]], w[p0 + e]);
+        __threadfence();
+        __syncthreads();
+        for (uint32_t s = threadIdx.x; s < cap; s += kLvThreads) {
+            const int C = __hip_atomic_load(&keys[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (C >= 0)
+                r.consider(C,
+                           __hip_atomic_load(&vals[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                           wtot, bs, bc, kcv);
+        }
     }
     wave_best(bs, bc);
     kcv = wave_max_u64(kcv);
-    const int wv = (int)(threadIdx.x >> 6);
-    if (lane_id() == 0) {
+    if (lane == 0) {
         rs[wv] = bs;
         rc[wv] = bc;
         rk[wv] = kcv;
@@ -263,9 +316,7 @@ k_move_heavy(const int32_t *heavy, const int64_t *ptr, const int32_t *adj, const
             best_merge(bs, bc, rs[i], rc[i]);
             kcv = rk[i] > kcv ? rk[i] : kcv;
         }
-        const int to = r.decide(bs, bc, kcv, wtot[cv], kvi);
-        cnew[v] = to;
-        if (to != cv) atomicAdd(moved, 1);
+        cnew[v] = r.decide(bs, bc, kcv, wtot[cv], kvi);
     }
 }
 
@@ -301,68 +352,117 @@ __global__ void k_wtot(int64_t n, const int32_t *c, const u64 *k, u64 *wtot) {
 }
 
 // totals after a sweep from those before it (wtot_new holds a copy): only
-// the nodes that moved change them (exact in two's-complement integers)
+// the nodes that moved change them (exact in two's-complement integers).  *moved
+// is set if any did, by one store per block: a counter or a flag that every move
+// writes serialises them.
 __global__ void k_wtot_moves(int64_t n, const int32_t *c, const int32_t *cnew, const u64 *k,
-                             u64 *wtot_new) {
+                             u64 *wtot_new, int *moved) {
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= n) return;
-    const int32_t a = c[v], b = cnew[v];
+    const int32_t a = v < n ? c[v] : 0, b = v < n ? cnew[v] : 0;
     if (a != b) {
         atomicAdd(&wtot_new[a], (u64)0 - k[v]);
         atomicAdd(&wtot_new[b], k[v]);
     }
+    if (__syncthreads_or(a != b) && threadIdx.x == 0)
+        __hip_atomic_store(moved, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// weight of the edges inside clusters (sum_w_in without tot_self), one
-// edge per thread over a fixed grid
-constexpr int kInBlocks = 2048;
+// After a sweep: the clustering and its totals are taken over (ACCEPT) or the
+// totals put back, so that wtot_new is a copy of wtot again.
+template <bool ACCEPT>
+__global__ void k_commit(int64_t n, int32_t *c, const int32_t *cnew, u64 *wtot, u64 *wtot_new) {
+    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= n) return;
+    if (ACCEPT) {
+        c[v] = cnew[v];
+        wtot[v] = wtot_new[v];
+    } else {
+        wtot_new[v] = wtot[v];
+    }
+}
+
+// The two sums of the modularity, by different blocks of one launch.
+// Blocks [0, kSqBlocks): sum over clusters of (w_tot / totw)^2 in a fixed order (a
+// fixed grid of strided partial sums, a fixed tree per block, then one block).
+// The others: weight of the edges inside clusters (sum_w_in without tot_self),
+// 4 edges at a time with all their gathers in flight; a partial sum per block, as
+// one shared accumulator takes the blocks' additions one after another.
+constexpr int kInBlocks = 1024;
+constexpr int kInEdges = 4;
+struct ModOut {
+    u64 in;
+    double sq;
+    int moved;
+};
 __global__ void __launch_bounds__(kLvThreads)
-k_mod_in(int64_t m, const int32_t *src, const int32_t *adj, const u64 *w, const int32_t *c,
-         u64 *acc) {
-    __shared__ u64 part[kLvWaves];
+k_mod_parts(int64_t L, const u64 *wtot, double totw, double *part, int64_t m, const int32_t *src,
+            const int32_t *adj, const u64 *w, const int32_t *c, u64 *ipart) {
+    if (blockIdx.x < kSqBlocks) {
+        __shared__ double sh[kLvThreads];
+        double s = 0.0;
+        for (int64_t i = (int64_t)blockIdx.x * kLvThreads + threadIdx.x; i < L;
+             i += (int64_t)kSqBlocks * kLvThreads) {
+            const double x = (double)wtot[i] / totw;
+            s += x * x;
+        }
+        sh[threadIdx.x] = s;
+        __syncthreads();
+        for (int o = kLvThreads / 2; o > 0; o >>= 1) {
+            if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+        return;
+    }
+    const int b = (int)blockIdx.x - kSqBlocks, nb = (int)gridDim.x - kSqBlocks;
     u64 s = 0;
-    for (int64_t e = (int64_t)blockIdx.x * kLvThreads + threadIdx.x; e < m;
-         e += (int64_t)kInBlocks * kLvThreads)
-        if (c[src[e]] == c[adj[e]]) s += w[e];
+    const int64_t m4 = m / kInEdges;
+    for (int64_t q = (int64_t)b * kLvThreads + threadIdx.x; q < m4; q += (int64_t)nb * kLvThreads) {
+        const int4 u = ((const int4 *)src)[q], v = ((const int4 *)adj)[q];
+        const ulonglong2 w0 = ((const ulonglong2 *)w)[2 * q], w1 = ((const ulonglong2 *)w)[2 * q + 1];
+        const int a0 = c[u.x], a1 = c[u.y], a2 = c[u.z], a3 = c[u.w];
+        const int b0 = c[v.x], b1 = c[v.y], b2 = c[v.z], b3 = c[v.w];
+        s += (a0 == b0 ? w0.x : 0) + (a1 == b1 ? w0.y : 0);
+        s += (a2 == b2 ? w1.x : 0) + (a3 == b3 ? w1.y : 0);
+    }
+    const int64_t e = kInEdges * m4 + threadIdx.x;
+    if (b == 0 && e < m && c[src[e]] == c[adj[e]]) s += w[e];
+    __shared__ u64 wpart[kLvWaves];
     s = wave_sum_u64(s);
-    if (lane_id() == 0) part[threadIdx.x >> 6] = s;
+    if (lane_id() == 0) wpart[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
         u64 t = 0;
-        for (int i = 0; i < kLvWaves; ++i) t += part[i];
-        if (t) atomicAdd(acc, t);
+        for (int i = 0; i < kLvWaves; ++i) t += wpart[i];
+        ipart[b] = t;
     }
 }
 
-// sum over clusters of (w_tot / totw)^2 in a fixed order: a fixed grid of
-// kSqBlocks strided partial sums, a fixed tree per block, then one block
+// Both sums and the flag of the sweep, which is cleared for the next one, to
+// host memory: the host reads them after one wait, without a copy.
 __global__ void __launch_bounds__(kLvThreads)
-k_mod_sq(int64_t L, const u64 *wtot, double totw, double *part) {
-    __shared__ double sh[kLvThreads];
-    double s = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * kLvThreads + threadIdx.x; i < L;
-         i += (int64_t)kSqBlocks * kLvThreads) {
-        const double x = (double)wtot[i] / totw;
-        s += x * x;
-    }
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = kLvThreads / 2; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
-__global__ void __launch_bounds__(kLvThreads) k_mod_sq_final(const double *part, double *out) {
+k_mod_final(const double *part, const u64 *ipart, int nb, int *moved, ModOut *out) {
+    static_assert(kSqBlocks == kLvThreads, "one partial sum per thread");
     __shared__ double sh[kSqBlocks];
+    __shared__ u64 wpart[kLvWaves];
     sh[threadIdx.x] = part[threadIdx.x];
+    u64 t = 0;
+    for (int i = threadIdx.x; i < nb; i += kLvThreads) t += ipart[i];
+    t = wave_sum_u64(t);
+    if (lane_id() == 0) wpart[threadIdx.x >> 6] = t;
     __syncthreads();
     for (int o = kSqBlocks / 2; o > 0; o >>= 1) {
         if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[0] = sh[0];
+    if (threadIdx.x == 0) {
+        t = 0;
+        for (int i = 0; i < kLvWaves; ++i) t += wpart[i];
+        out->in = t;
+        out->sq = sh[0];
+        out->moved = *moved;
+        *moved = 0;
+    }
 }
 
 // renumbering by first occurrence (renumber!, src/modularity.jl:289-315)
@@ -409,15 +509,10 @@ __global__ void k_merge(int64_t n, int32_t *c, const int32_t *cr) {
 }
 
 // reduced_network (src/modularity.jl:196-241): edge (c[u], c[v], w) keys
-__global__ void k_edge_keys(int64_t n, const int64_t *ptr, const int32_t *adj, const u64 *w,
-                            const int32_t *c, int b, u64 *key, u64 *val) {
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= n) return;
-    const u64 hi = (u64)c[v] << b;
-    for (int64_t e = ptr[v]; e < ptr[v + 1]; ++e) {
-        key[e] = hi | (u64)c[adj[e]];
-        val[e] = w[e];
-    }
+__global__ void k_edge_keys(int64_t m, const int32_t *src, const int32_t *adj, const int32_t *c,
+                            int b, u64 *key) {
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < m) key[e] = ((u64)c[src[e]] << b) | (u64)c[adj[e]];
 }
 
 // flag the first entry of each run of equal keys between distinct clusters
@@ -430,30 +525,58 @@ __global__ void k_run_heads(int64_t m, const u64 *key, int b, int32_t *flag) {
     flag[i] = (head && (kk >> b) != (kk & mask)) ? 1 : 0;
 }
 
+// Sums of the runs of equal keys: a run's entries in a wavefront are added up by
+// shuffles (the keys are sorted, so equal keys `o` lanes apart have only that key
+// between them) and one lane adds them to the run's total; the weight inside
+// clusters is kept per thread over a fixed grid.  One addition per entry and per
+// wavefront took 584 us for 2 million edges of 50,000 nodes, mostly waiting for
+// the same few addresses.
+constexpr int kEmitBlocks = 512;
 __global__ void __launch_bounds__(kLvThreads)
 k_run_emit(int64_t m, const u64 *key, const u64 *val, int b, const int32_t *flag,
            const int64_t *pos, int32_t *adj_r, int32_t *src_r, u64 *w_r, int32_t *rowcnt,
            u64 *self_acc) {
-    const int64_t i = (int64_t)blockIdx.x * kLvThreads + threadIdx.x;
+    const int lane = lane_id();
+    const u64 mask = (1ull << b) - 1ull;
     u64 self = 0;
-    if (i < m) {
-        const u64 kk = key[i];
-        const u64 mask = (1ull << b) - 1ull;
-        const u64 row = kk >> b, col = kk & mask;
-        if (row == col) {
-            self = val[i];
-        } else {
-            const int64_t g = pos[i] + flag[i] - 1;
-            if (flag[i]) {
-                adj_r[g] = (int32_t)col;
-                src_r[g] = (int32_t)row;
-                atomicAdd(&rowcnt[row], 1);
+    // whole wavefronts run every step (the base is the same in all lanes)
+    const int64_t step = (int64_t)gridDim.x * kLvThreads;
+    for (int64_t base = (int64_t)blockIdx.x * kLvThreads + threadIdx.x - lane; base < m;
+         base += step) {
+        const int64_t i = base + lane;
+        const u64 kk = i < m ? key[i] : ~0ull;
+        u64 t = i < m ? val[i] : 0;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const u64 ok = (u64)__shfl_down((long long)kk, o, kWave);
+            const u64 ot = (u64)__shfl_down((long long)t, o, kWave);
+            if (lane + o < kWave && ok == kk) t += ot;
+        }
+        const u64 prev = (u64)__shfl_up((long long)kk, 1, kWave);
+        if (i < m && (lane == 0 || prev != kk)) {
+            const u64 row = kk >> b, col = kk & mask;
+            if (row == col) {
+                self += t;
+            } else {
+                const int64_t g = pos[i] + flag[i] - 1;
+                if (flag[i]) {
+                    adj_r[g] = (int32_t)col;
+                    src_r[g] = (int32_t)row;
+                    atomicAdd(&rowcnt[row], 1);
+                }
+                atomicAdd(&w_r[g], t);
             }
-            atomicAdd(&w_r[g], val[i]);
         }
     }
+    __shared__ u64 wpart[kLvWaves];
     self = wave_sum_u64(self);
-    if (lane_id() == 0 && self) atomicAdd(self_acc, self);
+    if (lane == 0) wpart[threadIdx.x >> 6] = self;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        u64 t = 0;
+        for (int i = 0; i < kLvWaves; ++i) t += wpart[i];
+        if (t) atomicAdd(self_acc, t);
+    }
 }
 
 __global__ void k_set_i64(int64_t *a, int64_t val) { a[0] = val; }
@@ -489,11 +612,17 @@ __global__ void k_build_net(int64_t n, const int64_t *colptr, const int32_t *row
 }
 
 // largest weight as its bit pattern (ordered like the value for w >= 0)
+// (a fixed grid: one atomic per wavefront of the whole input took 0.7 ms)
+constexpr int kMaxBlocks = 512;
 template <class T>
 __global__ void __launch_bounds__(kLvThreads) k_max_bits(int64_t m, const T *val, u64 *acc) {
-    const int64_t i = (int64_t)blockIdx.x * kLvThreads + threadIdx.x;
-    const double x = i < m ? (double)val[i] : 0.0;
-    const u64 b = wave_max_u64((u64)__double_as_longlong(x));
+    u64 b = 0;
+    for (int64_t i = (int64_t)blockIdx.x * kLvThreads + threadIdx.x; i < m;
+         i += (int64_t)gridDim.x * kLvThreads) {
+        const u64 x = (u64)__double_as_longlong((double)val[i]);
+        b = x > b ? x : b;
+    }
+    b = wave_max_u64(b);
     if (lane_id() == 0 && b) atomicMax(acc, b);
 }
 
@@ -724,11 +853,12 @@ struct Louvain {
     std::vector<std::unique_ptr<LvLevel>> levels;  // stable addresses across depths
     // scratch shared by all depths (used within one phase at a time)
     DevBuf<int32_t> cnew, first, flag;
-    DevBuf<u64> wtot, wtot_new, key, val, key2, val2;
+    DevBuf<u64> wtot, wtot_new, key, key2, val2, ipart;
     DevBuf<int64_t> pos, scan_scratch;
-    DevBuf<int> hkeys, counter;
+    DevBuf<int> hkeys, counter, moved;
+    HostPinned<ModOut> out;
     DevBuf<u64> hvals, acc;
-    DevBuf<double> part, sq;
+    DevBuf<double> part;
     DevBuf<char> sort_tmp;
 
     int64_t scan_i32(const int32_t *in, int64_t n) {
@@ -764,24 +894,20 @@ struct Louvain {
         SEV_LAUNCH_CHECK();
     }
 
-    // modularity (src/modularity.jl:125-148) of clustering c with totals wt
+    // modularity (src/modularity.jl:125-148) of clustering c with totals wt;
+    // waits, and leaves the sweep's flag in out
     double modularity(const LvGraph &g, const int32_t *c, const u64 *wt) {
-        acc.ensure(1);
         part.ensure(kSqBlocks);
-        sq.ensure(1);
-        k_fill_u64<<<1, 1, 0, st>>>(acc.get(), 1, 0);
-        if (g.nnz > 0)
-            k_mod_in<<<(unsigned)std::min<int64_t>(kInBlocks, grid_of(g.nnz)), kLvThreads, 0, st>>>(
-                g.nnz, g.src.get(), g.adj.get(), g.w.get(), c, acc.get());
-        k_mod_sq<<<kSqBlocks, kLvThreads, 0, st>>>(g.n, wt, totw_d, part.get());
-        k_mod_sq_final<<<1, kSqBlocks, 0, st>>>(part.get(), sq.get());
+        ipart.ensure(kInBlocks);
+        ModOut *o = out.ensure(1);
+        const int nb = (int)std::min<int64_t>(kInBlocks, grid_of(g.nnz, kInEdges * kLvThreads));
+        k_mod_parts<<<(unsigned)(kSqBlocks + nb), kLvThreads, 0, st>>>(
+            g.n, wt, totw_d, part.get(), g.nnz, g.src.get(), g.adj.get(), g.w.get(), c,
+            ipart.get());
+        k_mod_final<<<1, kLvThreads, 0, st>>>(part.get(), ipart.get(), nb, moved.get(), o);
         SEV_LAUNCH_CHECK();
-        u64 in = 0;
-        double s = 0.0;
-        SEV_HIP(hipMemcpyAsync(&in, acc.get(), sizeof in, hipMemcpyDeviceToHost, st));
-        SEV_HIP(hipMemcpyAsync(&s, sq.get(), sizeof s, hipMemcpyDeviceToHost, st));
         SEV_HIP(hipStreamSynchronize(st));
-        return (double)(g.tot_self + in) / totw_d - res * s;
+        return (double)(g.tot_self + o->in) / totw_d - res * o->sq;
     }
 
     // local_move! (src/modularity.jl:255-287) in parallel sweeps; returns the
@@ -799,12 +925,14 @@ struct Louvain {
         cnew.ensure((size_t)n);
         wtot.ensure((size_t)n);
         wtot_new.ensure((size_t)n);
-        counter.ensure(1);
         if (g.nheavy > 0) {
             hkeys.ensure((size_t)(2 * g.nnz));
             hvals.ensure((size_t)(2 * g.nnz));
         }
         compute_wtot(g, c, wtot.get());
+        k_commit<false><<<grid_of(n), kLvThreads, 0, st>>>(n, c, cnew.get(), wtot.get(),
+                                                           wtot_new.get());
+        SEV_LAUNCH_CHECK();
         const double q0 = modularity(g, c, wtot.get());
         double q = q0, round_gain = 0.0;
         uint32_t athresh = kActAll >> 1;
@@ -815,36 +943,27 @@ struct Louvain {
                               0xD1B54A32D192ED03ull;
         for (int sweep = 0; sweep < kMaxSweeps; ++sweep) {
             const uint64_t akey = pkey + (uint64_t)sweep;
-            SEV_HIP(hipMemsetAsync(counter.get(), 0, sizeof(int), st));
-            k_move_light<2 * kSmallDeg><<<grid_of(n, kLvWaves), kLvThreads, 0, st>>>(
-                n, nullptr, g.ptr.get(), g.adj.get(), g.w.get(), g.k.get(), c, wtot.get(),
-                cnew.get(), totw_d, res, akey, athresh, counter.get());
-            if (g.nmedium > 0)
-                k_move_light<2 * kLightDeg><<<grid_of(g.nmedium, kLvWaves), kLvThreads, 0, st>>>(
-                    g.nmedium, g.medium.get(), g.ptr.get(), g.adj.get(), g.w.get(), g.k.get(), c,
-                    wtot.get(), cnew.get(), totw_d, res, akey, athresh, counter.get());
-            if (g.nheavy > 0)
-                k_move_heavy<<<(unsigned)g.nheavy, kLvThreads, 0, st>>>(
-                    g.heavy.get(), g.ptr.get(), g.adj.get(), g.w.get(), g.k.get(), c, wtot.get(),
-                    cnew.get(), hkeys.get(), hvals.get(), totw_d, res, akey, athresh,
-                    counter.get());
+            k_move_light<<<grid_of(n, kLvWaves), kLvThreads, 0, st>>>(
+                n, g.ptr.get(), g.adj.get(), g.w.get(), g.k.get(), c, wtot.get(), cnew.get(),
+                totw_d, res, akey, athresh);
+            if (g.nmedium > 0 || g.nheavy > 0)
+                k_move_large<<<(unsigned)(g.nheavy + ceil_div(g.nmedium, (int64_t)kLvWaves)),
+                               kLvThreads, 0, st>>>(
+                    g.heavy.get(), (int)g.nheavy, g.medium.get(), g.nmedium, g.ptr.get(),
+                    g.adj.get(), g.w.get(), g.k.get(), c, wtot.get(), cnew.get(), hkeys.get(),
+                    hvals.get(), totw_d, res, akey, athresh);
+            k_wtot_moves<<<grid_of(n), kLvThreads, 0, st>>>(n, c, cnew.get(), g.k.get(),
+                                                            wtot_new.get(), moved.get());
             SEV_LAUNCH_CHECK();
-            int moved = 0;
-            SEV_HIP(hipMemcpyAsync(&moved, counter.get(), sizeof moved, hipMemcpyDeviceToHost, st));
-            SEV_HIP(hipStreamSynchronize(st));
+            const double qn = modularity(g, cnew.get(), wtot_new.get());
             // a sweep in which no chosen node wants to move gains nothing; the
             // pair test below then ends the phase
-            if (moved != 0) {
-                SEV_HIP(hipMemcpyAsync(wtot_new.get(), wtot.get(), sizeof(u64) * (size_t)n,
-                                       hipMemcpyDeviceToDevice, st));
-                k_wtot_moves<<<grid_of(n), kLvThreads, 0, st>>>(n, c, cnew.get(), g.k.get(),
-                                                                wtot_new.get());
+            if (out.ptr->moved != 0) {
+                const auto commit = qn > q ? k_commit<true> : k_commit<false>;
+                commit<<<grid_of(n), kLvThreads, 0, st>>>(n, c, cnew.get(), wtot.get(),
+                                                          wtot_new.get());
                 SEV_LAUNCH_CHECK();
-                const double qn = modularity(g, cnew.get(), wtot_new.get());
                 if (qn > q) {
-                    SEV_HIP(hipMemcpyAsync(c, cnew.get(), sizeof(int32_t) * (size_t)n,
-                                           hipMemcpyDeviceToDevice, st));
-                    wtot.swap(wtot_new);
                     round_gain += qn - q;
                     q = qn;
                     athresh = kActAll >> 1;
@@ -903,18 +1022,17 @@ struct Louvain {
             return;
         }
         key.ensure((size_t)m);
-        val.ensure((size_t)m);
         key2.ensure((size_t)m);
         val2.ensure((size_t)m);
-        k_edge_keys<<<grid_of(g.n), kLvThreads, 0, st>>>(g.n, g.ptr.get(), g.adj.get(), g.w.get(),
-                                                         c, b, key.get(), val.get());
+        k_edge_keys<<<grid_of(m), kLvThreads, 0, st>>>(m, g.src.get(), g.adj.get(), c, b,
+                                                       key.get());
         SEV_LAUNCH_CHECK();
         size_t tb = 0;
-        SEV_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, key.get(), key2.get(), val.get(),
+        SEV_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, key.get(), key2.get(), g.w.get(),
                                                    val2.get(), (int)m, 0, 2 * b, st));
         sort_tmp.ensure(tb);
         SEV_HIP(hipcub::DeviceRadixSort::SortPairs(sort_tmp.get(), tb, key.get(), key2.get(),
-                                                   val.get(), val2.get(), (int)m, 0, 2 * b, st));
+                                                   g.w.get(), val2.get(), (int)m, 0, 2 * b, st));
         flag.ensure((size_t)m);
         k_run_heads<<<grid_of(m), kLvThreads, 0, st>>>(m, key2.get(), b, flag.get());
         SEV_LAUNCH_CHECK();
@@ -929,7 +1047,7 @@ struct Louvain {
         k_fill_u64<<<grid_of(ne), kLvThreads, 0, st>>>(r.w.get(), ne, 0);
         k_fill_i32<<<grid_of(nc), kLvThreads, 0, st>>>(rowcnt.get(), nc, 0);
         k_fill_u64<<<1, 1, 0, st>>>(acc.get(), 1, 0);
-        k_run_emit<<<grid_of(m), kLvThreads, 0, st>>>(m, key2.get(), val2.get(), b, flag.get(),
+        k_run_emit<<<std::min<unsigned>(kEmitBlocks, grid_of(m)), kLvThreads, 0, st>>>(m, key2.get(), val2.get(), b, flag.get(),
                                                       pos.get(), r.adj.get(), r.src.get(),
                                                       r.w.get(), rowcnt.get(), acc.get());
         SEV_LAUNCH_CHECK();
@@ -985,7 +1103,7 @@ int64_t louvain_cluster(int64_t n, const int64_t *colptr_d, const int32_t *row_d
                                                           val64.get());
             val_d = val64.get();
         }
-        k_max_bits<<<grid_of(nnz), kLvThreads, 0, st>>>(nnz, val_d, mx.get());
+        k_max_bits<<<std::min<unsigned>(kMaxBlocks, grid_of(nnz)), kLvThreads, 0, st>>>(nnz, val_d, mx.get());
         SEV_LAUNCH_CHECK();
         SEV_HIP(hipMemcpyAsync(&maxbits, mx.get(), sizeof maxbits, hipMemcpyDeviceToHost, st));
         SEV_HIP(hipStreamSynchronize(st));
@@ -1029,6 +1147,8 @@ int64_t louvain_cluster(int64_t n, const int64_t *colptr_d, const int32_t *row_d
                                                        std::ldexp(1.0, S), g.ptr.get(),
                                                        g.adj.get(), g.src.get(), g.w.get(),
                                                        g.k.get());
+        lv.moved.ensure(1);
+        k_fill_i32<<<1, 1, 0, st>>>(lv.moved.get(), 1, 0);
         lv.acc.ensure(1);
         k_fill_u64<<<1, 1, 0, st>>>(lv.acc.get(), 1, 0);
         k_sum_u64<<<grid_of(n), kLvThreads, 0, st>>>(n, g.k.get(), lv.acc.get());

@@ -254,3 +254,26 @@ def test_full_size_properties(sev, orc):
     print(f"1M cells: {lab.max()} clusters, modularity {q:.6f} (oracle on the labels {qo:.6f})")
     assert q == pytest.approx(qo, abs=1e-9)
     assert adjusted_rand_score(centre, lab) > 0.99
+
+
+@pytest.mark.parametrize("d", [1, 3, 64, 65, 128, 129, 256, 257, 1024, 1025])
+def test_degree_edges_of_the_move_kernels(sev, d):
+    """Two complete graphs of degree d joined by one link (an edge count that is
+    no multiple of 4): the degrees at which a node changes from a wavefront to a
+    block and from LDS to global tables.  Both are recovered and the modularity
+    is that of the labels (1e-9: fixed point of 2^-40)."""
+    rng = np.random.default_rng(d)
+    n = d + 1
+    A = np.zeros((2 * n, 2 * n))
+    for b in range(2):
+        U = np.triu(rng.uniform(0.5, 1.0, (n, n)), 1)
+        A[b * n:(b + 1) * n, b * n:(b + 1) * n] = U + U.T
+    A[0, n] = A[n, 0] = 0.01
+    lab, q = sev.cluster(sp.csc_matrix(A), resolution=1.0, return_modularity=True,
+                         group_singletons=False)
+    block = np.repeat([0, 1], n)
+    assert adjusted_rand_score(block, lab) == 1.0
+    k, tot = A.sum(axis=0), A.sum()
+    want = sum(A[np.ix_(lab == c, lab == c)].sum() / tot - (k[lab == c].sum() / tot) ** 2
+               for c in np.unique(lab))
+    assert abs(q - want) < 1e-9
