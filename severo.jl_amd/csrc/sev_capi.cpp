@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstring>
 #include <limits>
@@ -262,6 +263,141 @@ void download(T *h, const T *d, size_t n, hipStream_t st) {
     if (n) SEV_HIP(hipMemcpyAsync(h, d, sizeof(T) * n, hipMemcpyDeviceToHost, st));
 }
 
+// Device-to-host transfer of large results.  A copy into pageable memory is staged
+// by the runtime in one thread, at about 10 GB/s into pages that were never touched
+// (the arrays a caller has just allocated); here the DMA fills pinned slots in turn
+// and a few threads take each slot over as it lands, converting as they copy.  The
+// slots belong to one pipeline, are allocated at its first large result and are
+// given back with it.
+struct DownStage {
+    static constexpr int kSlots = 4;
+    static constexpr size_t kBytes = (size_t)8 << 20;  // per slot
+    static constexpr int kThreads = 8;
+    HostPinned<char> buf;
+    hipEvent_t landed[kSlots] = {};
+    DownStage() = default;
+    DownStage(const DownStage &) = delete;
+    DownStage &operator=(const DownStage &) = delete;
+    ~DownStage() {
+        for (hipEvent_t e : landed)
+            if (e) (void)hipEventDestroy(e);
+    }
+    void ensure() {
+        buf.ensure(kSlots * kBytes);
+        for (hipEvent_t &e : landed)
+            if (!e) SEV_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+};
+
+// from here on the slots are faster than the runtime's staging, their threads
+// and events included
+constexpr size_t kDownMinBytes = (size_t)32 << 20;
+
+// take(in, first, count): elements [first, first + count) of src are at in; called
+// from several threads at once, with first and count in multiples of unit (but for
+// the end).  Returns when all are taken.
+template <class S, class F>
+void staged_download(DownStage &ds, const S *src, int64_t n, int64_t unit, F &&take,
+                     hipStream_t st) {
+    ds.ensure();
+    const int64_t per =
+        std::max<int64_t>(1, (int64_t)(DownStage::kBytes / sizeof(S)) / unit) * unit;
+    SEV_REQUIRE((size_t)per * sizeof(S) <= DownStage::kBytes, "download unit too large");
+    const int64_t nc = ceil_div(n, per);
+    const int nt = (int)std::max<unsigned>(
+        1, std::min<unsigned>(std::thread::hardware_concurrency(), DownStage::kThreads));
+    auto slot = [&](int64_t c) {
+        return (S *)(ds.buf.ptr + (size_t)(c % DownStage::kSlots) * DownStage::kBytes);
+    };
+    struct Team {
+        std::mutex mu;
+        std::condition_variable cv;
+        int64_t ready = 0;      // chunks that have landed
+        bool stop = false;      // none will land any more
+        std::vector<int> left;  // threads that have not taken their part of a chunk
+        std::vector<std::thread> th;
+        ~Team() {
+            {
+                std::lock_guard<std::mutex> l(mu);
+                stop = true;
+            }
+            cv.notify_all();
+            for (auto &x : th) x.join();
+        }
+    } team;
+    team.left.assign((size_t)nc, nt);
+    auto work = [&](int t) {
+        for (int64_t c = 0; c < nc; ++c) {
+            {
+                std::unique_lock<std::mutex> l(team.mu);
+                team.cv.wait(l, [&] { return team.ready > c || team.stop; });
+                if (team.ready <= c) return;
+            }
+            const int64_t p0 = c * per, len = std::min<int64_t>(per, n - p0);
+            const int64_t units = ceil_div(len, unit);
+            const int64_t a = std::min<int64_t>(len, units * t / nt * unit);
+            const int64_t b = std::min<int64_t>(len, units * (t + 1) / nt * unit);
+            if (a < b) take((const S *)slot(c) + a, p0 + a, b - a);
+            std::lock_guard<std::mutex> l(team.mu);
+            if (--team.left[(size_t)c] == 0) team.cv.notify_all();
+        }
+    };
+    for (int t = 0; t < nt; ++t) team.th.emplace_back(work, t);
+    auto taken = [&](int64_t c) {
+        std::unique_lock<std::mutex> l(team.mu);
+        team.cv.wait(l, [&] { return team.left[(size_t)c] == 0; });
+    };
+    int64_t issued = 0;
+    try {
+        for (int64_t c = 0; c < nc; ++c) {
+            for (; issued < nc && issued < c + DownStage::kSlots; ++issued) {
+                if (issued >= DownStage::kSlots) taken(issued - DownStage::kSlots);
+                const int64_t p0 = issued * per, len = std::min<int64_t>(per, n - p0);
+                SEV_HIP(hipMemcpyAsync(slot(issued), src + p0, sizeof(S) * (size_t)len,
+                                       hipMemcpyDeviceToHost, st));
+                SEV_HIP(hipEventRecord(ds.landed[issued % DownStage::kSlots], st));
+            }
+            SEV_HIP(hipEventSynchronize(ds.landed[c % DownStage::kSlots]));
+            {
+                std::lock_guard<std::mutex> l(team.mu);
+                team.ready = c + 1;
+            }
+            team.cv.notify_all();
+        }
+        taken(nc - 1);
+    } catch (...) {
+        (void)hipStreamSynchronize(st);  // no copy into the slots stays in flight
+        throw;
+    }
+}
+
+// n elements to h, by either way
+template <class T>
+void download_large(DownStage &ds, T *h, const T *d, size_t n, hipStream_t st) {
+    if (n * sizeof(T) < kDownMinBytes) return download(h, d, n, st);
+    staged_download(
+        ds, d, (int64_t)n, 1,
+        [h](const T *in, int64_t first, int64_t count) {
+            std::memcpy(h + first, in, sizeof(T) * (size_t)count);
+        },
+        st);
+}
+
+// n 0-based int32 indexes to 1-based int64
+void download_index(DownStage &ds, int64_t *h, const int32_t *d, int64_t n, hipStream_t st) {
+    auto take = [h](const int32_t *in, int64_t first, int64_t count) {
+        for (int64_t i = 0; i < count; ++i) h[first + i] = (int64_t)in[i] + 1;
+    };
+    if ((size_t)n * sizeof(int32_t) >= kDownMinBytes) {
+        staged_download(ds, d, n, 1, take, st);
+    } else {
+        std::vector<int32_t> rv((size_t)n);
+        download(rv.data(), d, rv.size(), st);
+        SEV_HIP(hipStreamSynchronize(st));
+        take(rv.data(), 0, n);
+    }
+}
+
 // xmin and weight table for the Jaccard graph: w[x] = x/(k + (k - x)) in T,
 // keep iff |w| > T(prune) (droptol!).
 template <class T>
@@ -287,6 +423,7 @@ int snn_table(int64_t k, double prune, std::vector<T> &w) {
 struct sev_pipeline {
     Stream stream;
     Prof prof;
+    DownStage down;  // large results to the host
     // counts (cells x genes CSC)
     int64_t m = 0, g = 0, nnz = 0;
     DevBuf<int64_t> cp;
@@ -690,15 +827,12 @@ int sev_pipeline_get_counts(sev_pipeline *p, int64_t *colptr, int64_t *rowval, i
         ProfInstall pi_(&p->prof);
         SEV_REQUIRE(p->have_counts, "no counts loaded");
         hipStream_t st = p->st();
-        std::vector<int32_t> rv((size_t)p->nnz);
         if (colptr) download(colptr, p->cp.get(), (size_t)p->g + 1, st);
-        if (rowval) download(rv.data(), p->row.get(), (size_t)p->nnz, st);
-        if (nzval) download(nzval, p->cnt.get(), (size_t)p->nnz, st);
+        if (rowval) download_index(p->down, rowval, p->row.get(), p->nnz, st);
+        if (nzval) download_large(p->down, nzval, p->cnt.get(), (size_t)p->nnz, st);
         SEV_HIP(hipStreamSynchronize(st));
         if (colptr)
             for (int64_t j = 0; j <= p->g; ++j) colptr[j] += 1;
-        if (rowval)
-            for (int64_t i = 0; i < p->nnz; ++i) rowval[i] = (int64_t)rv[(size_t)i] + 1;
     });
 }
 
@@ -723,7 +857,7 @@ int sev_pipeline_get_normalized(sev_pipeline *p, float *nzval) {
     return guarded([&] {
         ProfInstall pi_(&p->prof);
         SEV_REQUIRE(p->have_norm, "normalize has not run");
-        download(nzval, p->norm.get(), (size_t)p->nnz, p->st());
+        download_large(p->down, nzval, p->norm.get(), (size_t)p->nnz, p->st());
         SEV_HIP(hipStreamSynchronize(p->st()));
     });
 }
@@ -943,9 +1077,9 @@ int sev_pipeline_get_pca(sev_pipeline *p, double *s, double *U, double *V, float
         hipStream_t st = p->st();
         const int64_t S = p->nsamples();
         if (s) std::memcpy(s, p->s.data(), sizeof(double) * (size_t)(S * p->npcs));
-        if (U) download(U, p->U.get(), (size_t)(p->m * p->npcs), st);
-        if (V) download(V, p->V.get(), (size_t)(S * p->F * p->npcs), st);
-        if (Z) download(Z, p->Z.get(), (size_t)(p->m * p->npcs), st);
+        if (U) download_large(p->down, U, p->U.get(), (size_t)(p->m * p->npcs), st);
+        if (V) download_large(p->down, V, p->V.get(), (size_t)(S * p->F * p->npcs), st);
+        if (Z) download_large(p->down, Z, p->Z.get(), (size_t)(p->m * p->npcs), st);
         SEV_HIP(hipStreamSynchronize(st));
     });
 }
@@ -1093,6 +1227,28 @@ int sev_pipeline_get_neighbours(sev_pipeline *p, int32_t *nn_index, float *dista
         SEV_REQUIRE(p->have_nn, "neighbours have not run");
         hipStream_t st = p->st();
         const int64_t m = p->m, k = p->k;
+        // rows of k to columns of m
+        if ((size_t)(m * k) * sizeof(int32_t) >= kDownMinBytes) {
+            if (nn_index)
+                staged_download(
+                    p->down, p->nn.get(), m * k, k,
+                    [=](const int32_t *in, int64_t first, int64_t count) {
+                        for (int64_t t = 0; t < k; ++t)
+                            for (int64_t i = 0; i < count / k; ++i)
+                                nn_index[first / k + i + t * m] = in[i * k + t] + 1;
+                    },
+                    st);
+            if (distances)
+                staged_download(
+                    p->down, p->dist.get(), m * k, k,
+                    [=](const float *in, int64_t first, int64_t count) {
+                        for (int64_t t = 0; t < k; ++t)
+                            for (int64_t i = 0; i < count / k; ++i)
+                                distances[first / k + i + t * m] = in[i * k + t];
+                    },
+                    st);
+            return;
+        }
         std::vector<int32_t> idx((size_t)(m * k));
         std::vector<float> dd((size_t)(m * k));
         download(idx.data(), p->nn.get(), idx.size(), st);
@@ -1215,20 +1371,17 @@ int sev_pipeline_get_snn(sev_pipeline *p, int64_t *colptr, int64_t *rowval, void
         SEV_REQUIRE(p->have_snn, "snn has not run");
         hipStream_t st = p->st();
         const int64_t m = p->m, nnz = p->snn_nnz;
-        std::vector<int32_t> rv((size_t)nnz);
         if (colptr) download(colptr, p->scp.get(), (size_t)m + 1, st);
-        if (rowval) download(rv.data(), p->srow.get(), (size_t)nnz, st);
+        if (rowval) download_index(p->down, rowval, p->srow.get(), nnz, st);
         if (nzval) {
             if (p->snn_dtype == SEV_FLOAT32)
-                download((float *)nzval, p->sval32.get(), (size_t)nnz, st);
+                download_large(p->down, (float *)nzval, p->sval32.get(), (size_t)nnz, st);
             else
-                download((double *)nzval, p->sval64.get(), (size_t)nnz, st);
+                download_large(p->down, (double *)nzval, p->sval64.get(), (size_t)nnz, st);
         }
         SEV_HIP(hipStreamSynchronize(st));
         if (colptr)
             for (int64_t j = 0; j <= m; ++j) colptr[j] += 1;
-        if (rowval)
-            for (int64_t i = 0; i < nnz; ++i) rowval[i] = (int64_t)rv[(size_t)i] + 1;
     });
 }
 

@@ -231,3 +231,25 @@ def test_pipeline_neighbours_cosine(sev, orc, precision):
     cp, rv, nz = orc.snn(ridx, 15, 1 / 15, np.float32)
     assert np.array_equal(S.indptr, cp - 1) and np.array_equal(S.data, nz)
     p.close()
+
+
+def test_large_results_in_slots(sev):
+    """Results large enough to come through the pinned slots (from 32 MiB; sizes
+    that are no multiple of a slot) equal the one-shot calls', which copy
+    directly."""
+    rng = np.random.default_rng(5)
+    m, k = 420_011, 20
+    Z = np.asfortranarray(rng.standard_normal((m, 3)).astype(np.float32))
+    p = sev.Pipeline()
+    p.set_embedding(Z)
+    p.neighbours(k, include_self=True)
+    idx, dist = p.get_neighbours(m)
+    ridx, rdist = sev.ann(Z, k)
+    assert np.array_equal(idx, ridx) and np.array_equal(dist, rdist)
+    p.snn(1 / 15, np.float32)
+    S = p.get_snn(m)
+    assert S.nnz * 4 >= 32 << 20
+    R = sev.shared_nearest_neighbours(Z, k)
+    assert np.array_equal(S.indptr, R.indptr) and np.array_equal(S.indices, R.indices)
+    assert np.array_equal(S.data, R.data)
+    p.close()
