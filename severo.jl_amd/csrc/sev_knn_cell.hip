@@ -76,6 +76,10 @@ constexpr int kPivLd = 64;        // floats per pivot row (zero padded)
 constexpr int kSample = 16384;    // points of the Lloyd steps
 constexpr int kTestPivots = 1024; // structure test: pivots and queries
 constexpr int kTestQueries = 256;
+// Bound of the error of nq - 2 s from the norm's three parts: a part below 2^-14
+// is taken as zero, once (2^-13), whatever the scale.  It matters where the scale
+// stops at 2^60 (largest |z| below 2e-18) and the relative terms vanish.
+constexpr double kNormErr = 0x1p-12;
 
 // FP16 bits of x, 0 below the normal range
 __device__ __forceinline__ uint16_t f2h(float x) {
@@ -679,13 +683,13 @@ k_knn_cell(CellArgs a) {
         // distance at most U^2 / spec
         const double dt = nq - 2.0 * (double)sv;
         const double U = sqrt((dt > 0.0 ? dt : 0.0) * (1.0 + 0x1p-21) + a.eta * (nq + ncmax) +
-                              1e-30) + eq + emax;
+                              kNormErr) + eq + emax;
         const bool live = a.perm[q0 + row] >= 0;
         // a group is out of reach when nq - 2 s > (T + R)^2 with room for the
         // score's error
         float T = (float)((U / a.spec + eq) * (1.0 + 1e-5));
         if (!(sv > -6e4f) || !(T == T)) T = __builtin_huge_valf();
-        float A = (float)(nq - (1.02 * a.eta + 4e-6) * (nq + nbmax));
+        float A = (float)(nq - (1.02 * a.eta + 4e-6) * (nq + nbmax) - kNormErr);
         L.thr[row] = live ? T : 0.0f;
         L.ta[row] = live ? A : __builtin_huge_valf();
     });
@@ -870,7 +874,7 @@ k_cell_rerank(const T *Zs, const int32_t *perm, const int *tot, int d, int k,
     const double nq = (double)nhat[s];
     const double dt = nq - 2.0 * (double)cthr[s];
     const double lb2 = dt * (1.0 - 0x1p-21) -
-                       eta * (nq + (double)__uint_as_float(gmax[0])) - 1e-30;
+                       eta * (nq + (double)__uint_as_float(gmax[0])) - kNormErr;
     const double lb = lb2 > 0.0 ? sqrt(lb2) - (double)eps[s] - (double)__uint_as_float(gmax[1])
                                 : -1.0;
     const double sc = (double)point_scale(gmax[3]);

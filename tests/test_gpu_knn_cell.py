@@ -70,3 +70,18 @@ def test_exhaustive_head_bound(sev, orc, dtype, n, d, k):
                             precision="exact")
         ridx, rdist = orc.knn(np.asfortranarray(X), kk, include_self=include_self)
         assert np.array_equal(idx, ridx) and np.array_equal(dist, rdist)
+
+
+@pytest.mark.parametrize("scale", [1e-18, 3e-19])
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+def test_cells_tiny_values(sev, orc, precision, scale):
+    """Coordinates so small that the operands' scale stops at 2^60: the parts of
+    the norms that are taken as zero then weigh as much as the gaps between
+    neighbours, and rows must not be certified on them."""
+    rng = np.random.default_rng(17)
+    n, d = 12500, 20
+    X = rng.normal(0, 0.3, (12, d))[rng.integers(0, 12, n)] + rng.normal(0, 0.02, (n, d))
+    X = np.asfortranarray((X * scale).astype(np.float32))
+    idx, dist = sev.ann(X, 10, precision=precision)
+    ridx, rdist = orc.knn(X, 10)
+    assert np.array_equal(idx, ridx) and np.array_equal(dist, rdist)
