@@ -1341,9 +1341,15 @@ void knn_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int i
                 run_mfma<0, 128, 1, 32, 128>(Z, n, d, ld, k, include_self, w, idx, dist, st,
                                              n_fallback, rows);
             } else {
-                // wide rows with long lists exceed the LDS budget: exhaustive
-                knn_exact<float>(Z, n, d, ld, k, include_self, nullptr, n, idx, dist, st);
-                if (n_fallback) *n_fallback = n;
+                // wide rows with long lists exceed the LDS budget: exhaustive, for
+                // the rows that the cells left (60,000 x 55, k = 28: 6.0 ms, all rows
+                // 28) or for all
+                if (rows >= 0)
+                    knn_exact_rows<float>(Z, n, d, ld, k, include_self, w.fail.get(), rows, idx,
+                                          dist, st);
+                else
+                    knn_exact<float>(Z, n, d, ld, k, include_self, nullptr, n, idx, dist, st);
+                if (n_fallback) *n_fallback = rows >= 0 ? rows : n;
             }
         }
     }

@@ -85,3 +85,17 @@ def test_cells_tiny_values(sev, orc, precision, scale):
     idx, dist = sev.ann(X, 10, precision=precision)
     ridx, rdist = orc.knn(X, 10)
     assert np.array_equal(idx, ridx) and np.array_equal(dist, rdist)
+
+
+def test_cells_wide_rows_left(sev, orc):
+    """FP32, 52 <= d <= 63 and k > 24: no matrix-core lists exist for the rows
+    that the cells leave without a certificate (among them a block of points
+    with more equal distances than a list holds), and only those rows are
+    searched exhaustively."""
+    n, d, k = 12500, 55, 30
+    X = _points(n, d, 20, seed=55)
+    X[100:200] = X[100]
+    idx, dist, left = sev.ann(X, k, return_fallback=True)
+    ridx, rdist = orc.knn(X, k)
+    assert np.array_equal(idx, ridx) and np.array_equal(dist, rdist)
+    assert 100 <= left < n // 2
