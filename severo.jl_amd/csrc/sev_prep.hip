@@ -312,6 +312,14 @@ struct WelfordChunk {
     T v[kWave], F[kWave], y[kWave];
 };
 
+// Orders a wavefront's LDS accesses across its lanes (its LDS operations are
+// carried out in order: this only keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // mu and s of the column whose entry p < e has the value value(p), the count
 // starting at count (before the first entry).
 template <class T, class V>
@@ -331,6 +339,7 @@ __device__ __forceinline__ void welford_column(int64_t b, int64_t e, int64_t cou
         L.v[lane] = vl;
         L.F[lane] = Fl;
         L.y[lane] = welford_rcp(Fl);
+        wave_lds_sync();
         const bool plain = __all(!(lane < nt) || vl >= welford_floor<T>()) &&
                            mu >= welford_floor<T>();
         if (plain && nt == kWave) {
@@ -368,6 +377,7 @@ __device__ __forceinline__ void welford_column(int64_t b, int64_t e, int64_t cou
             }
         }
         count += nt;
+        wave_lds_sync();  // the chunk is overwritten next
     }
     mu_ = mu;
     s_ = s;

@@ -224,3 +224,20 @@ def test_scale_stats_chunk_edges(sev, orc, dt, n):
     C = sev.scale_features(A, scale_max=10.0, dtype=dt)
     B, mu, _ = orc.scale(m, A.indptr.astype(np.int64), A.data, dt(10.0))
     assert np.array_equal(C.A.data, B, equal_nan=True) and np.array_equal(C.mu, mu, equal_nan=True)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_scale_stats_many_chunks(sev, orc, dt):
+    """Columns of many chunks, every wavefront of several blocks at work, each
+    chunk with values of its own size: what one lane puts in LDS for a chunk is
+    what all lanes read for it, and nothing of the chunk before or after."""
+    rng = np.random.default_rng(64)
+    m, cols = 9000, 37
+    nnz = [int(x) for x in rng.integers(4000, 9000, cols)]
+    data = [(rng.lognormal(0, 1, n) * 10.0 ** (np.arange(n) // 64 % 5)).astype(dt) for n in nnz]
+    rows = np.concatenate([np.sort(rng.choice(m, n, replace=False)) for n in nnz])
+    A = sp.csc_matrix((np.concatenate(data), rows, np.concatenate([[0], np.cumsum(nnz)])),
+                      shape=(m, cols))
+    C = sev.scale_features(A, scale_max=10.0, dtype=dt)
+    B, mu, _ = orc.scale(m, A.indptr.astype(np.int64), A.data, dt(10.0))
+    assert np.array_equal(C.A.data, B) and np.array_equal(C.mu, mu)
