@@ -10,6 +10,8 @@
 // correctly rounded operations.
 #include "sev_kernels.hpp"
 
+#include <type_traits>
+
 namespace sev {
 
 namespace {
@@ -275,9 +277,13 @@ k_gather_copy(const int64_t *feat, const int64_t *colptr, const int32_t *row, co
 //    stalled it: 83 cycles per step in FP32, now 45; in FP64 with the division
 //    300, now 112);
 //  - whether a quotient could leave the normal range is decided per chunk, from
-//    the chunk's smallest value and mu: values and means of at least 2^-60
-//    (FP64: 2^-400) differ by zero or by 2^-84 (2^-453) or more.  Other chunks
-//    take the division itself.
+//    the chunk's values and mu: finite values and means of at least 2^-60 (FP64:
+//    2^-400) differ by zero or by 2^-84 (2^-453) or more.  Chunks with stored
+//    zeros or negative values, and those of fewer than 64 entries, note tiny
+//    differences beside the chain, and are done again with the division itself if
+//    there was one or a value was not finite (300 columns of 120,000 entries, 30%
+//    stored zeros: with the division at once 5.8 ms in FP32, now 3.5; 20,000 of 50
+//    entries: 0.038 against 0.021).
 // 1M cells, the 2,000 variable genes (FP32): 32.2 -> 17.6 ms; 27,998 genes'
 // counts (FP64): 116 -> 43.5 ms.
 // --------------------------------------------------------------------------
@@ -304,6 +310,20 @@ __device__ __forceinline__ double welford_rcp(double F) { return 1.0 / F; }
 template <class T>
 __device__ __forceinline__ T welford_floor() {
     return sizeof(T) == 4 ? (T)0x1p-60 : (T)0x1p-400;
+}
+// welford_floor <= x, finite (the bits of positive values order as integers)
+__device__ __forceinline__ bool welford_plain(float x) {
+    return __float_as_uint(x) - 0x21800000u < 0x7f800000u - 0x21800000u;
+}
+__device__ __forceinline__ bool welford_plain(double x) {
+    const uint32_t h = (uint32_t)((uint64_t)__double_as_longlong(x) >> 32);
+    return h - 0x26f00000u < 0x7ff00000u - 0x26f00000u;
+}
+// a difference whose remainder could leave the normal range
+template <class T>
+__device__ __forceinline__ bool welford_tiny(T delta) {
+    const T lo = sizeof(T) == 4 ? (T)0x1p-90 : (T)0x1p-900;
+    return (int)(fabs(delta) < lo) & (int)(delta != T(0));
 }
 
 // A wavefront's chunk: values, counts and reciprocals of 64 steps.
@@ -340,12 +360,13 @@ __device__ __forceinline__ void welford_column(int64_t b, int64_t e, int64_t cou
         L.F[lane] = Fl;
         L.y[lane] = welford_rcp(Fl);
         wave_lds_sync();
-        const bool plain = __all(!(lane < nt) || vl >= welford_floor<T>()) &&
-                           mu >= welford_floor<T>();
-        if (plain && nt == kWave) {
-            // groups of 8 steps, the next group's operands read from LDS
-            // while the chain runs over the current ones
-            constexpr int U = 8;
+        // groups of U steps, the next group's operands read from LDS while the
+        // chain runs over the current ones.  full: 64 steps; check: tiny
+        // differences are noted beside the chain, and false is returned if there
+        // was one, or if anything was not finite (mu and s are then void).
+        auto chain = [&](auto full_, auto check_, int nt) -> bool {
+            constexpr bool kFull = decltype(full_)::value, kCheck = decltype(check_)::value;
+            constexpr int U = sizeof(T) == 8 ? 4 : 8;  // (8 in FP64: over 128 registers)
             T v[2][U], F[2][U], y[2][U];
             auto take = [&](int g, T (&v)[U], T (&F)[U], T (&y)[U]) {
 #pragma unroll
@@ -355,25 +376,42 @@ __device__ __forceinline__ void welford_column(int64_t b, int64_t e, int64_t cou
 #pragma unroll
                 for (int u = 0; u < U; ++u) y[u] = L.y[g * U + u];
             };
+            bool tiny = false;
             take(0, v[0], F[0], y[0]);
 #pragma unroll
             for (int g = 0; g < kWave / U; ++g) {
+                if (!kFull && g * U >= nt) break;
                 if (g + 1 < kWave / U) take(g + 1, v[(g + 1) & 1], F[(g + 1) & 1], y[(g + 1) & 1]);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
+                    if (!kFull && g * U + u >= nt) break;
                     const T x = v[g & 1][u], delta = x - mu;
+                    if (kCheck) tiny |= welford_tiny(delta);
                     mu = mu + welford_quot(delta, F[g & 1][u], y[g & 1][u]);
                     s = s + delta * (x - mu);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
+            return !tiny && mu - mu == T(0);
+        };
+        const bool plain = nt == kWave && mu >= welford_floor<T>() && __all(welford_plain(vl));
+        if (plain) {
+            (void)chain(std::true_type(), std::false_type(), kWave);
         } else {
-            for (int t = 0; t < nt; ++t) {
-                const T v = L.v[t];
-                const T delta = v - mu;
-                mu = mu + delta / L.F[t];
-                s = s + delta * (v - mu);
+            const T mu0 = mu, s0 = s;
+            const bool ok = nt == kWave ? chain(std::true_type(), std::true_type(), kWave)
+                                        : chain(std::false_type(), std::true_type(),
+                                                __builtin_amdgcn_readfirstlane(nt));
+            if (__builtin_expect(!__all(ok), 0)) {
+                mu = mu0;
+                s = s0;
+                for (int t = 0; t < nt; ++t) {
+                    const T v = L.v[t];
+                    const T delta = v - mu;
+                    mu = mu + delta / L.F[t];
+                    s = s + delta * (v - mu);
+                }
             }
         }
         count += nt;
@@ -429,7 +467,7 @@ k_scale_stats_lane(int64_t ncol, const int64_t *colptr, const float *x, float sc
         const float F = (float)count, y = welford_rcp(F);
         const float delta = v - mu;
         float q = welford_quot(delta, F, y);
-        if (fabsf(delta) < 0x1p-90f && delta != 0.0f) q = delta / F;
+        if (welford_tiny(delta)) q = delta / F;
         mu = mu + q;
         s = s + delta * (v - mu);
     };

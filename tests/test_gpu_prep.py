@@ -241,3 +241,30 @@ def test_scale_stats_many_chunks(sev, orc, dt):
     C = sev.scale_features(A, scale_max=10.0, dtype=dt)
     B, mu, _ = orc.scale(m, A.indptr.astype(np.int64), A.data, dt(10.0))
     assert np.array_equal(C.A.data, B) and np.array_equal(C.mu, mu)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [5, 63, 64, 65, 200, 640])
+def test_scale_stats_out_of_range_chunks(sev, orc, dt, n):
+    """Columns whose chunks are checked step by step (stored zeros, negative
+    values, fewer than 64 entries), with differences that fall below the range
+    of the quotient's correction step or above it in some chunks: sd and mu' bit
+    for bit as the oracle's sequential recurrence."""
+    rng = np.random.default_rng(n)
+    m, cols = n, 9  # no unstored entries: the mean starts at the first value
+    tiny, huge = (1e-36, 3e37) if dt == np.float32 else (1e-290, 1e307)
+    data = rng.lognormal(0, 1, (cols, n))
+    data[0, rng.random(n) < 0.3] = 0.0
+    data[1] *= np.where(rng.random(n) < 0.5, 1.0, -1.0)
+    data[2] = tiny * rng.random(n)
+    data[3, n // 2:] = tiny
+    data[4] = 1.0 + np.finfo(dt).eps * rng.integers(0, 3, n)
+    data[5] = 0.0
+    data[6] = np.where(rng.random(n) < 0.5, huge, -huge)
+    data[7, n // 2] = np.inf
+    data[8] = huge * rng.random(n)
+    A = sp.csc_matrix((data.astype(dt).ravel(), np.tile(np.arange(n), cols),
+                       np.arange(cols + 1) * n), shape=(m, cols))
+    C = sev.scale_features(A, scale_max=10.0, dtype=dt)
+    B, mu, _ = orc.scale(m, A.indptr.astype(np.int64), A.data, dt(10.0))
+    assert np.array_equal(C.A.data, B, equal_nan=True) and np.array_equal(C.mu, mu, equal_nan=True)
