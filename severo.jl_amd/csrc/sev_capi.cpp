@@ -9,7 +9,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <condition_variable>
 #include <cstdio>
 #include <cstring>
 #include <limits>
@@ -20,6 +19,7 @@
 
 #include "../../include/severo_hip.h"
 #include "sev_kernels.hpp"
+#include "sev_team.hpp"
 
 #include <atomic>
 
@@ -282,10 +282,17 @@ struct DownStage {
         for (hipEvent_t e : landed)
             if (e) (void)hipEventDestroy(e);
     }
-    void ensure() {
-        buf.ensure(kSlots * kBytes);
-        for (hipEvent_t &e : landed)
-            if (!e) SEV_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    // false: no pinned memory or events to be had
+    bool ensure() {
+        try {
+            buf.ensure(kSlots * kBytes);
+            for (hipEvent_t &e : landed)
+                if (!e) SEV_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            return true;
+        } catch (...) {
+            (void)hipGetLastError();
+            return false;
+        }
     }
 };
 
@@ -295,76 +302,53 @@ constexpr size_t kDownMinBytes = (size_t)32 << 20;
 
 // take(in, first, count): elements [first, first + count) of src are at in; called
 // from several threads at once, with first and count in multiples of unit (but for
-// the end).  Returns when all are taken.
+// the end).  Returns when all are taken.  Without pinned memory the chunks come
+// through pageable memory, without threads they are taken by the caller's.
 template <class S, class F>
 void staged_download(DownStage &ds, const S *src, int64_t n, int64_t unit, F &&take,
                      hipStream_t st) {
-    ds.ensure();
     const int64_t per =
         std::max<int64_t>(1, (int64_t)(DownStage::kBytes / sizeof(S)) / unit) * unit;
     SEV_REQUIRE((size_t)per * sizeof(S) <= DownStage::kBytes, "download unit too large");
     const int64_t nc = ceil_div(n, per);
-    const int nt = (int)std::max<unsigned>(
-        1, std::min<unsigned>(std::thread::hardware_concurrency(), DownStage::kThreads));
+    auto fetch = [&](int64_t c, S *h) {
+        const int64_t p0 = c * per, len = std::min<int64_t>(per, n - p0);
+        SEV_HIP(hipMemcpyAsync(h, src + p0, sizeof(S) * (size_t)len, hipMemcpyDeviceToHost, st));
+    };
+    if (!ds.ensure()) {
+        std::vector<S> h((size_t)std::min<int64_t>(per, n));
+        for (int64_t c = 0; c < nc; ++c) {
+            fetch(c, h.data());
+            SEV_HIP(hipStreamSynchronize(st));
+            take((const S *)h.data(), c * per, std::min<int64_t>(per, n - c * per));
+        }
+        return;
+    }
     auto slot = [&](int64_t c) {
         return (S *)(ds.buf.ptr + (size_t)(c % DownStage::kSlots) * DownStage::kBytes);
     };
-    struct Team {
-        std::mutex mu;
-        std::condition_variable cv;
-        int64_t ready = 0;      // chunks that have landed
-        bool stop = false;      // none will land any more
-        std::vector<int> left;  // threads that have not taken their part of a chunk
-        std::vector<std::thread> th;
-        ~Team() {
-            {
-                std::lock_guard<std::mutex> l(mu);
-                stop = true;
-            }
-            cv.notify_all();
-            for (auto &x : th) x.join();
-        }
-    } team;
-    team.left.assign((size_t)nc, nt);
-    auto work = [&](int t) {
-        for (int64_t c = 0; c < nc; ++c) {
-            {
-                std::unique_lock<std::mutex> l(team.mu);
-                team.cv.wait(l, [&] { return team.ready > c || team.stop; });
-                if (team.ready <= c) return;
-            }
+    ChunkTeam<> team(
+        (int)std::max<unsigned>(
+            1, std::min<unsigned>(std::thread::hardware_concurrency(), DownStage::kThreads)),
+        nc, [&](int64_t c, int t, int nt) {
             const int64_t p0 = c * per, len = std::min<int64_t>(per, n - p0);
             const int64_t units = ceil_div(len, unit);
             const int64_t a = std::min<int64_t>(len, units * t / nt * unit);
             const int64_t b = std::min<int64_t>(len, units * (t + 1) / nt * unit);
             if (a < b) take((const S *)slot(c) + a, p0 + a, b - a);
-            std::lock_guard<std::mutex> l(team.mu);
-            if (--team.left[(size_t)c] == 0) team.cv.notify_all();
-        }
-    };
-    for (int t = 0; t < nt; ++t) team.th.emplace_back(work, t);
-    auto taken = [&](int64_t c) {
-        std::unique_lock<std::mutex> l(team.mu);
-        team.cv.wait(l, [&] { return team.left[(size_t)c] == 0; });
-    };
+        });
     int64_t issued = 0;
     try {
         for (int64_t c = 0; c < nc; ++c) {
             for (; issued < nc && issued < c + DownStage::kSlots; ++issued) {
-                if (issued >= DownStage::kSlots) taken(issued - DownStage::kSlots);
-                const int64_t p0 = issued * per, len = std::min<int64_t>(per, n - p0);
-                SEV_HIP(hipMemcpyAsync(slot(issued), src + p0, sizeof(S) * (size_t)len,
-                                       hipMemcpyDeviceToHost, st));
+                if (issued >= DownStage::kSlots) team.wait(issued - DownStage::kSlots);
+                fetch(issued, slot(issued));
                 SEV_HIP(hipEventRecord(ds.landed[issued % DownStage::kSlots], st));
             }
             SEV_HIP(hipEventSynchronize(ds.landed[c % DownStage::kSlots]));
-            {
-                std::lock_guard<std::mutex> l(team.mu);
-                team.ready = c + 1;
-            }
-            team.cv.notify_all();
+            team.publish(c);
         }
-        taken(nc - 1);
+        team.wait(nc - 1);
     } catch (...) {
         (void)hipStreamSynchronize(st);  // no copy into the slots stays in flight
         throw;
@@ -374,6 +358,7 @@ void staged_download(DownStage &ds, const S *src, int64_t n, int64_t unit, F &&t
 // n elements to h, by either way
 template <class T>
 void download_large(DownStage &ds, T *h, const T *d, size_t n, hipStream_t st) {
+    SEV_REQUIRE(n == 0 || h != nullptr, "output is NULL");
     if (n * sizeof(T) < kDownMinBytes) return download(h, d, n, st);
     staged_download(
         ds, d, (int64_t)n, 1,

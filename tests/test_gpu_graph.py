@@ -253,3 +253,22 @@ def test_large_results_in_slots(sev):
     assert np.array_equal(S.indptr, R.indptr) and np.array_equal(S.indices, R.indices)
     assert np.array_equal(S.data, R.data)
     p.close()
+
+
+def test_large_result_to_null_is_refused(sev):
+    """A result above the size that comes through the pinned slots, asked for
+    without an array to put it in, is an error as a small one is."""
+    import scipy.sparse as sp
+    m, n = 500_000, 18
+    rng = np.random.default_rng(2)
+    X = sp.csc_matrix((rng.integers(1, 9, m * n).astype(np.int32), np.tile(np.arange(m), n),
+                       np.arange(n + 1) * m), shape=(m, n))
+    p = sev.Pipeline()
+    p.load_counts(X)
+    p.normalize("lognormalize", 1e4)
+    assert m * n * 4 >= 32 << 20
+    L = sev.load()
+    assert L.sev_pipeline_get_normalized(p._h, None) == -1
+    assert b"NULL" in L.sev_last_error()
+    assert len(p.get_normalized()) == m * n
+    p.close()
