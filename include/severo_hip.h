@@ -199,12 +199,16 @@ void FindNeighboursCosine32(const float *X, int n, int d, int ld, int k, int nta
 void FindNeighboursCosine64(const double *X, int n, int d, int ld, int k, int ntables,
                             int include_self, int seed, int32_t *nn_index, double *distances);
 
-/* Same search with a status and a precision form: SEV_PREC_FP32 (FP32
- * candidates on MFMA), SEV_PREC_BF16 (BF16 candidates on MFMA) -- both
- * followed by an exact FP32 re-rank and a certificate, so the result equals
- * the exact search -- or SEV_PREC_EXACT (exhaustive).  Float64 input always
- * uses the exhaustive search.  *n_fallback (may be NULL) receives the number
- * of query rows that were recomputed exhaustively. */
+/* Same search with a status and a precision form.  Every form returns the
+ * exact result: neighbours are ranked by distances in the precision of X, and
+ * a row is taken from candidates only if a bound certifies it.  SEV_PREC_EXACT
+ * always searches exhaustively, SEV_PREC_FP32 and SEV_PREC_BF16 choose the way
+ * by the shape: few points exhaustively, otherwise matrix-core candidates over
+ * cells of nearby points (FP16 operands; two parts each for SEV_PREC_FP32 and
+ * for Float64 input) or over all points (FP32 or BF16 operands).  *n_fallback
+ * (may be NULL) receives the number of query rows that were searched
+ * exhaustively: those that no candidates could certify, or all n where the
+ * search was exhaustive from the start. */
 int sev_knn(const void *X, int64_t n, int64_t d, int64_t ld, int dtype, int64_t k,
             int include_self, int precision, int32_t *nn_index, void *distances,
             int64_t *n_fallback);
@@ -395,8 +399,9 @@ int sev_pipeline_get_pca(sev_pipeline *p, double *s, double *U, double *V, float
 int sev_pipeline_set_embedding(sev_pipeline *p, int64_t m, int64_t d, const float *Z, int64_t ld);
 
 /* Stage 4: exact kNN on the first ndims embedding dimensions (ndims <= 0:
- * all).  For a batch, the neighbours of a cell are cells of its own sample
- * (indices stay those of the stacked rows). */
+ * all), in the forms of sev_knn (and *n_fallback as there).  For a batch, the
+ * neighbours of a cell are cells of its own sample (indices stay those of the
+ * stacked rows). */
 int sev_pipeline_neighbours(sev_pipeline *p, int64_t k, int include_self, int64_t ndims,
                             int precision, int64_t *n_fallback);
 /* The same with metric=CosineDist() (src/neighbours.jl:159-204): the search

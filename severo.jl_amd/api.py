@@ -420,7 +420,8 @@ def ann(X, k: int, include_self=True, ntables=None, precision="fp32", return_fal
     1-based Int32, distances n x k), column-major like the reference.
     ``precision`` selects how candidates are proposed ("fp32" / "bf16"
     matrix cores with an exact re-rank, or "exact" exhaustive); the result is
-    the same.  ``metric="cosine"`` (Distances.CosineDist) searches the rows
+    the same.  ``return_fallback`` adds the number of rows searched
+    exhaustively (all of them where there are few points).  ``metric="cosine"`` (Distances.CosineDist) searches the rows
     scaled to unit length and reports D / 2 of the unit rows (1 - cos in
     exact arithmetic)."""
     X = np.asfortranarray(X)

@@ -418,10 +418,11 @@ void knn_exact_rows_batch(const float *X, int64_t n, int64_t d, int64_t ld, int6
                           const int32_t *row_sample, int32_t *idx, float *dist, hipStream_t st);
 
 // ---- sev_knn_mfma.hip ----------------------------------------------------
-// The same exact kNN (FP32 definition) by MFMA candidate search (FP32 or
-// BF16 operands), exact FP32 re-rank and a certificate; uncertified rows are
-// recomputed exhaustively.  Z is n x d column-major (ld).  Outputs row-major
-// n x k, 0-based.  *n_fallback = rows recomputed exhaustively.
+// The same exact kNN (FP32 definition): exhaustively for few points, otherwise
+// by MFMA candidates (over cells, sev_knn_cell.hip, or over all points in FP32
+// or BF16), exact FP32 re-rank and a certificate; uncertified rows are searched
+// exhaustively.  Z is n x d column-major (ld).  Outputs row-major n x k,
+// 0-based.  *n_fallback = rows searched exhaustively.
 struct KnnWork {
     DevBuf<unsigned char> zq, zc, zcp, stmp;
     DevBuf<float> zr, nhat, eps, cthr, pval, pthr, scf, hn;

@@ -1297,7 +1297,7 @@ void knn_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int i
     // below 8.0; 40,000: 10.6 against 10.3).
     if ((n * d <= 400000 && n <= 12000) || (!cells && n <= 30000)) {
         knn_exact<float>(Z, n, d, ld, k, include_self, nullptr, n, idx, dist, st);
-        if (n_fallback) *n_fallback = 0;
+        if (n_fallback) *n_fallback = n;
         return;
     }
     if (cells) {

@@ -272,3 +272,26 @@ def test_large_result_to_null_is_refused(sev):
     assert b"NULL" in L.sev_last_error()
     assert len(p.get_normalized()) == m * n
     p.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_fallback_counts_rows_searched_exhaustively(sev, dtype):
+    """n_fallback is n wherever the whole search is exhaustive (few points, the
+    exact form), and the rows left without a certificate (here few or none)
+    where candidates are proposed."""
+    rng = np.random.default_rng(3)
+    def points(n, d):
+        return np.asfortranarray((rng.normal(0, 6, (9, d))[rng.integers(0, 9, n)] +
+                                  rng.normal(0, 1, (n, d))).astype(dtype))
+    for n, d, precision in ((900, 8, "fp32"), (900, 8, "bf16"), (5000, 50, "fp32"),
+                            (20000, 10, "exact")):
+        assert sev.ann(points(n, d), 10, precision=precision, return_fallback=True)[2] == n
+    for precision in ("fp32", "bf16"):
+        assert sev.ann(points(20000, 20), 10, precision=precision, return_fallback=True)[2] < 200
+    if dtype == np.float32:
+        p = sev.Pipeline()
+        p.set_embedding(points(900, 8))
+        assert p.neighbours(10) == 900
+        p.set_embedding(points(20000, 20))
+        assert p.neighbours(10) < 200
+        p.close()
