@@ -515,7 +515,7 @@ void knn_host(const T *X, int64_t n, int64_t d, int64_t ld, int64_t k, int inclu
         KnnWork w;
         knn_mfma((const float *)dx.get(), n, d, n, k, include_self, precision == SEV_PREC_BF16, w,
                  idx.get(), (float *)dist.get(), s.st, &nfb);
-    } else if (sizeof(T) == 8 && precision != SEV_PREC_EXACT && knn_cell_f64_pays(n, d) &&
+    } else if (sizeof(T) == 8 && precision != SEV_PREC_EXACT && knn_cell_f64_pays(n, d, k) &&
                knn_cell_fits(n, d, k)) {
         KnnWork w;
         knn_cell_f64((const double *)dx.get(), n, d, n, k, include_self, w, idx.get(),

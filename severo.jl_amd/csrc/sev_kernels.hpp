@@ -441,12 +441,28 @@ struct KnnWork {
 // FP32 form (operands in two FP16 parts); otherwise one part, and -1 is
 // returned (nothing written) when the points have no clusters to skip.
 // Returns the rows without a certificate (their numbers in w.fail).
-constexpr int64_t kCellMinPoints = 4096;
 constexpr double kCellMaxShare = 0.4;
-// FP64 points: by cells above these sizes (one call on host arrays: 15,000 x
-// 50: 2.6 ms, exhaustively 3.2; 10,000 x 50: 2.3 against 1.9; 20,011 x 15: 1.6
-// against 1.8; 15,000 x 15: 1.4 against 1.2)
-inline bool knn_cell_f64_pays(int64_t n, int64_t d) { return n > 18000 || n * d > 600000; }
+// Rank past the k-th neighbour that bounds a list: the further, the wider the
+// gap that certifies a row; a list of 64 holds rank 34 (48 expected) and, at 2%
+// overflows, rank 36.
+inline int knn_cell_rank(int64_t k) { return (int)(k <= 24 ? k + 10 : k + 6); }
+// From rank 32 on a few rows in ten thousand overflow: enough for the search of
+// the rows left, a fixed cost, to run on most calls.
+inline bool knn_cell_leaves_rows(int64_t k) { return knn_cell_rank(k) >= 32; }
+// What the exhaustive kernel's time goes with: 8 operations or so per pair beside
+// those of the coordinates.
+inline double knn_pair_work(int64_t n, int64_t d) {
+    return (double)n * (double)n * (double)(d + 8);
+}
+// FP64 points: by cells above this work, or more where rows are left.  One call
+// on host arrays, exhaustively against by cells, for points in 12 groups and
+// without any: 20,000 x 10, k = 10: 1.35 against 1.39 and 1.76 ms; 20,011 x 15: 1.8
+// against 1.6; 26,000 x 10: 1.9 against 1.5 and 2.1; 16,000 x 50: 3.0 against 2.4
+// and 2.5; k = 24: 20,000 x 20: 2.6 against 2.2 and 2.9; 12,500 x 60: 2.9 against
+// 3.2 and 3.5; 26,000 x 20: 3.8 against 2.6 and 3.4.
+inline bool knn_cell_f64_pays(int64_t n, int64_t d, int64_t k) {
+    return knn_pair_work(n, d) > (knn_cell_leaves_rows(k) ? 1.35e10 : 8.5e9);
+}
 bool knn_cell_fits(int64_t n, int64_t d, int64_t k);
 template <class T>
 int64_t knn_cell(const T *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,

@@ -929,9 +929,7 @@ void run_cell(int64_t n, int64_t d, int64_t k, int include_self, int M, KnnWork 
     a.tot = tot;
     a.include_self = include_self;
     a.rank_k = (int)k;
-    // the further past k, the wider the gap that certifies a row; a list of
-    // 64 holds rank 34 (48 expected) and, at 2% overflows, rank 36
-    a.rank_l = k <= 24 ? (int)k + 10 : (int)k + 6;
+    a.rank_l = knn_cell_rank(k);
     // FP32 accumulation over KP terms, the dropped l.l' (2^-22) and the
     // three-part norm
     a.eta = 4.0 * (KP + 2) * 0x1p-24 + 0x1p-20;
@@ -961,8 +959,7 @@ void run_cell(int64_t n, int64_t d, int64_t k, int include_self, int M, KnnWork 
 bool knn_cell_fits(int64_t n, int64_t d, int64_t k) {
     // at k = 30 a list of 64 overflows for 2% of the rows; 3 d + 3 operand
     // columns of at most 192
-    return n >= kCellMinPoints && n <= (int64_t)kGrp * (kMaxGroups - kMaxPivots - 64) && k <= 30 &&
-           d <= 63;
+    return n <= (int64_t)kGrp * (kMaxGroups - kMaxPivots - 64) && k <= 30 && d <= 63;
 }
 
 template <class T>

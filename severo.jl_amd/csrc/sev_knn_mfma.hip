@@ -1278,6 +1278,37 @@ void knn_mfma_fp8(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, i
     }
 }
 
+// Where the exhaustive kernel is the fastest way (its time hardly depends on the
+// points or k).  The lines lie where it is no slower than
+// the other ways, for points without groups against the lists over all points;
+// for points in groups it is then far ahead of those.  Times in ms of the search
+// alone, exhaustively against:
+//  - cells, 12 groups, k = 20: 12,500 x 10 0.30 against 0.82, 16,000 x 20 0.68
+//    against 0.75, 20,000 x 20 0.93 against 0.72, 9,000 x 50 0.55 against 0.77,
+//    12,500 x 50 0.89 against 0.87.  Where the cells leave rows (k = 24): 16,000 x
+//    50 1.35 against 1.77, 20,000 x 50 1.94 against 1.49; and in FP32 from 52
+//    dimensions on with k > 24, where no lists exist for those rows, 16,000 x 60,
+//    k = 30 1.55 against 2.74 without groups and 1.96 with;
+//  - lists, no groups, up to 51 dimensions and k = 31: 30,000 x 51 4.1 against 4.5
+//    (30,000 x 15 1.5 against 5.1); k = 45: 20,000 x 51 1.9 against 2.0, 30,000 x 51
+//    4.2 against 3.8; from k = 49 on the lists of 64 certify ever fewer rows (k =
+//    64 none: 4.5 against 22.8);
+//  - FP32 lists, 64 to 127 dimensions: 30,000 x 64 4.9 against 6.6, 25,000 x 80 4.8
+//    against 5.1, 20,000 x 100 3.5 against 4.1, 25,000 x 100 6.0 against 5.1, 16,000
+//    x 126 3.2 against 3.3;
+//  - BF16 lists, 52 to 126 dimensions: 16,000 x 60 1.62 against 1.68, 20,000 x 60
+//    2.4 against 1.9, 12,000 x 100 1.4 against 1.8, 16,000 x 100 2.5 against 1.8.
+static bool exhaustive_pays(int64_t n, int64_t d, int64_t k, bool bf16, bool cells) {
+    const double nd = (double)n * (double)d, w = knn_pair_work(n, d);
+    const bool no_lists = !bf16 && d > 51 && k > 24;
+    if (cells) return w <= (no_lists ? 1.8e10 : (knn_cell_leaves_rows(k) ? 1.5e10 : 8.8e9));
+    if (no_lists) return true;
+    if (n > 30000) return false;
+    if (k > 48) return true;
+    if (d <= 51) return k <= 40 || nd <= 1.1e6;
+    return bf16 ? w <= 1.65e10 : nd <= 2.0e6;
+}
+
 void knn_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
               int bf16, KnnWork &w, int32_t *idx, float *dist, hipStream_t st,
               int64_t *n_fallback) {
@@ -1290,12 +1321,7 @@ void knn_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int i
         SEV_REQUIRE(d + 1 <= 128, "knn: FP32 MFMA form supports d <= 127");
     int64_t rows = -1;
     const bool cells = knn_cell_fits(n, d, k);
-    // Small searches are fastest exhaustively: at d = 50 up to 8,000 points
-    // (7,000: 0.60 ms, by cells 0.79; 10,000: 0.91 against 0.85-0.92), at d = 15
-    // up to 12,000 (10,000: 0.35 against 0.66; 15,000: 0.71 against 0.74); where
-    // cells do not apply up to 30,000 (d = 50: 6.0 ms, by the candidate lists
-    // below 8.0; 40,000: 10.6 against 10.3).
-    if ((n * d <= 400000 && n <= 12000) || (!cells && n <= 30000)) {
+    if (exhaustive_pays(n, d, k, bf16, cells)) {
         knn_exact<float>(Z, n, d, ld, k, include_self, nullptr, n, idx, dist, st);
         if (n_fallback) *n_fallback = n;
         return;
@@ -1341,15 +1367,12 @@ void knn_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int i
                 run_mfma<0, 128, 1, 32, 128>(Z, n, d, ld, k, include_self, w, idx, dist, st,
                                              n_fallback, rows);
             } else {
-                // wide rows with long lists exceed the LDS budget: exhaustive, for
-                // the rows that the cells left (60,000 x 55, k = 28: 6.0 ms, all rows
-                // 28) or for all
-                if (rows >= 0)
-                    knn_exact_rows<float>(Z, n, d, ld, k, include_self, w.fail.get(), rows, idx,
-                                          dist, st);
-                else
-                    knn_exact<float>(Z, n, d, ld, k, include_self, nullptr, n, idx, dist, st);
-                if (n_fallback) *n_fallback = rows >= 0 ? rows : n;
+                // wide rows with long lists exceed the LDS budget: the rows that
+                // the cells left go on exhaustively (60,000 x 55, k = 28: 6.0 ms,
+                // all rows 28)
+                knn_exact_rows<float>(Z, n, d, ld, k, include_self, w.fail.get(), rows, idx, dist,
+                                      st);
+                if (n_fallback) *n_fallback = rows;
             }
         }
     }

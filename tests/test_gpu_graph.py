@@ -175,11 +175,10 @@ def test_ann_mfma_duplicates(sev, orc):
 @pytest.mark.parametrize("precision", ["fp32", "bf16"])
 @pytest.mark.parametrize("include_self", [True, False])
 def test_ann_norm_order_ties(sev, orc, precision, include_self):
-    """Candidates searched by ascending norm with seeded thresholds (enough
-    points for a seeded head): exact duplicates, copies with the coordinates
-    reversed (equal norms, other points) and a block of zero vectors at the
-    head of the order.  The lists depend on the order only through ties, and
-    the certified result must not."""
+    """Exact duplicates, copies with the coordinates reversed (equal norms,
+    other points) and a block of zero vectors.  (Few points: searched
+    exhaustively; the lists in norm order meet the same ties in
+    test_lists_over_all_points.)"""
     rng = np.random.default_rng(31)
     base = rng.standard_normal((3000, 16)).astype(np.float32)
     X = np.concatenate([base, base[:, ::-1], base[:2000], np.zeros((50, 16), np.float32)])
@@ -284,7 +283,7 @@ def test_fallback_counts_rows_searched_exhaustively(sev, dtype):
         return np.asfortranarray((rng.normal(0, 6, (9, d))[rng.integers(0, 9, n)] +
                                   rng.normal(0, 1, (n, d))).astype(dtype))
     for n, d, precision in ((900, 8, "fp32"), (900, 8, "bf16"), (5000, 50, "fp32"),
-                            (20000, 10, "exact")):
+                            (20000, 20, "exact")):
         assert sev.ann(points(n, d), 10, precision=precision, return_fallback=True)[2] == n
     for precision in ("fp32", "bf16"):
         assert sev.ann(points(20000, 20), 10, precision=precision, return_fallback=True)[2] < 200
@@ -295,3 +294,43 @@ def test_fallback_counts_rows_searched_exhaustively(sev, dtype):
         p.set_embedding(points(20000, 20))
         assert p.neighbours(10) < 200
         p.close()
+
+
+@pytest.mark.parametrize("include_self", [True, False])
+@pytest.mark.parametrize("n,d,k,precision",
+                         [(30100, 16, 40, "fp32"), (30100, 16, 40, "bf16"),
+                          (30100, 51, 31, "fp32"), (30100, 51, 31, "bf16"),
+                          (30100, 20, 45, "fp32"), (30100, 20, 45, "bf16"),
+                          (15900, 126, 20, "fp32"), (11300, 126, 20, "bf16"),
+                          (15900, 70, 40, "bf16"), (30500, 16, 20, "bf16"),
+                          (16800, 52, 12, "bf16")])
+def test_lists_over_all_points(sev, orc, n, d, k, precision, include_self):
+    """The candidate lists over all points (sizes beyond the exhaustive search
+    that the cells do not take, or points without clusters in the BF16 form),
+    in ascending norm with seeded thresholds: exact duplicates, copies with the
+    coordinates reversed (equal norms, other points) and a block of zero
+    vectors at the head of the order.  The lists depend on the order only
+    through ties, and the certified result must not.  All rows against the
+    exhaustive form, 1,500 of them against the oracle."""
+    rng = np.random.default_rng(n + d)
+    u = n // 3
+    z = 40 if d < 60 else 10  # in many dimensions they are near every point
+    base = rng.standard_normal((u, d)).astype(np.float32)
+    X = np.concatenate([base, base[:, ::-1], base[:n - 2 * u - z],
+                        np.zeros((z, d), np.float32)])
+    X = np.asfortranarray(X)
+    p = sev.Pipeline()
+    p.set_embedding(X)
+    p.profile(True)
+    left = p.neighbours(k, include_self=include_self, precision=precision)
+    idx, dist = p.get_neighbours(n)
+    ran = set(p.profile_read())
+    assert "knn_cell" not in ran and left < n
+    assert any(r.startswith("knn_cand_" + precision) for r in ran)
+    p.neighbours(k, include_self=include_self, precision="exact")
+    xidx, xdist = p.get_neighbours(n)
+    p.close()
+    assert np.array_equal(idx, xidx) and np.array_equal(dist, xdist)
+    q = np.sort(np.concatenate([rng.choice(n - 40, 1460, replace=False), np.arange(n - 40, n)]))
+    ridx, rdist = orc.knn(X, k, include_self=include_self, qidx=q)
+    assert np.array_equal(idx[q], ridx) and np.array_equal(dist[q], rdist)
