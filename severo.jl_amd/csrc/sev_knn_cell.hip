@@ -14,13 +14,16 @@
 // ones: 7% of the groups at 1,000,000 x 50 with 40 clusters, 11% at 100,000
 // with 24 (40% with sampled points as centroids, which miss small clusters).
 //
-// Operands.  z is scaled by a power of two (largest |z|^2 in (2^12, 2^14]) and
-// rounded to FP16, relative error 2^-12 where BF16 has 2^-9, at the same rate:
+// Operands.  z is taken around the mean of a sample (the error of a score goes
+// with the norms: 100,000 x 50, 300 from the origin, 24 groups, FP32: 70 ms, most
+// rows without a certificate; now 2.1), scaled by a power of two (largest |z|^2 in
+// (2^12, 2^14]) and rounded to FP16, relative error 2^-11 where BF16 has 2^-8, at
+// the same rate:
 // with BF16 the rounding exceeds the gap between the k-th neighbour and the
 // end of the list wherever clusters lie far from the origin, and nearly every
 // row lost its certificate (1,000,000 x 50, 40 clusters: a first pass of 251 ms,
 // then 263 ms for the rows left).  The FP32 form splits z into two FP16 parts
-// h + l (2^-23) and takes q.c as h.h' + l.h' + h.l': three products at a sixth of
+// h + l (2^-22) and takes q.c as h.h' + l.h' + h.l': three products at a sixth of
 // the time of one on the FP32 matrix instruction.  FP16 parts below the
 // normal range are taken as zero, so their treatment by the MFMA does not
 // matter.
@@ -100,10 +103,34 @@ __device__ __forceinline__ float point_scale(unsigned n2) {
     return ldexpf(1.0f, e > 60 ? 60 : (e < -60 ? -60 : e));
 }
 
-// Zr[i*d + t] = Z[t*ld + i], 64 points per block through LDS; n2 = max |z|^2
+// cen[t] = mean of coordinate t over sampled points (0 if not finite), one block
+// per coordinate; gmax[0..3] = 0.
 template <class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_rows(const T *Z, int64_t n, int d, int64_t ld, T *Zr, unsigned *n2) {
+k_cell_centre(const T *Z, int64_t n, int64_t ld, float *cen, unsigned *gmax) {
+    __shared__ double part[kNW];
+    const int t = blockIdx.x;
+    if (t == 0 && threadIdx.x < 4) gmax[threadIdx.x] = 0u;
+    double a = 0.0;
+#pragma unroll
+    for (int u = 0; u < kTestPivots / kBlock; ++u)
+        a += (double)Z[t * ld + (int64_t)(threadIdx.x + u * kBlock) * n / kTestPivots];
+    a = wave_sum(a);
+    if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = a;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const float m = (float)((part[0] + part[1] + part[2] + part[3]) / kTestPivots);
+    cen[t] = fabsf(m) < __builtin_huge_valf() ? m : 0.0f;
+}
+
+// z - cen rounded to FP32
+__device__ __forceinline__ float centred(float z, float c) { return z - c; }
+__device__ __forceinline__ float centred(double z, float c) { return (float)(z - (double)c); }
+
+// Zr[i*d + t] = Z[t*ld + i], 64 points per block through LDS; n2 = max |z - cen|^2
+template <class T>
+__global__ void __launch_bounds__(kBlock)
+k_cell_rows(const T *Z, int64_t n, int d, int64_t ld, const float *cen, T *Zr, unsigned *n2) {
     __shared__ T s[kWave * 65];
     __shared__ float nn[kNW][kWave];
     const int64_t i0 = (int64_t)blockIdx.x * kWave;
@@ -114,7 +141,8 @@ k_cell_rows(const T *Z, int64_t n, int d, int64_t ld, T *Zr, unsigned *n2) {
         if (lane < nr) {
             const T z = Z[(int64_t)t * ld + i0 + lane];
             s[lane * (d + 1) + t] = z;
-            a = fmaf((float)z, (float)z, a);
+            const float zc = centred(z, cen[t]);
+            a = fmaf(zc, zc, a);
         }
     nn[w][lane] = a;
     __syncthreads();
@@ -128,25 +156,26 @@ k_cell_rows(const T *Z, int64_t n, int d, int64_t ld, T *Zr, unsigned *n2) {
     }
 }
 
-// piv[m*kPivLd + t] = coordinates of the point (m * n) / M, zero padded
+// piv[m*kPivLd + t] = centred coordinates of the point (m * n) / M, zero padded
 template <class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_pivots(const T *Zr, int64_t n, int d, int M, float *piv) {
+k_cell_pivots(const T *Zr, const float *cen, int64_t n, int d, int M, float *piv) {
     for (int e = blockIdx.x * kBlock + threadIdx.x; e < M * kPivLd; e += gridDim.x * kBlock) {
         const int m = e / kPivLd, t = e % kPivLd;
-        piv[e] = t < d ? (float)Zr[((int64_t)m * n / M) * d + t] : 0.0f;
+        piv[e] = t < d ? centred(Zr[((int64_t)m * n / M) * d + t], cen[t]) : 0.0f;
     }
 }
 
-// S[t*ns + i] = coordinates of the point (i * n) / ns; coordinate t of point j at
-// X[j*ri + t*rt].  *zero (if given) is set to 0.
+// S[t*ns + i] = coordinates of the point (i * n) / ns (less cen, if given);
+// coordinate t of point j at X[j*ri + t*rt].  *zero (if given) is set to 0.
 template <class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_sample(const T *X, int64_t ri, int64_t rt, int64_t n, int d, int ns, float *S, int *zero) {
+k_cell_sample(const T *X, int64_t ri, int64_t rt, const float *cen, int64_t n, int d, int ns,
+              float *S, int *zero) {
     if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
     for (int e = blockIdx.x * kBlock + threadIdx.x; e < ns * d; e += gridDim.x * kBlock) {
         const int t = e / ns, i = e % ns;
-        S[e] = (float)X[((int64_t)i * n / ns) * ri + t * rt];
+        S[e] = centred(X[((int64_t)i * n / ns) * ri + t * rt], cen ? cen[t] : 0.0f);
     }
 }
 
@@ -280,7 +309,8 @@ k_cell_order(const float *piv, const float *half, int M, int d, float *out, floa
 // addresses, so they reach the FMAs as scalar operands.
 template <int DP, class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_assign(const T *Z, int64_t n, int d, int64_t ld, const float *__restrict__ piv,
+k_cell_assign(const T *Z, int64_t n, int d, int64_t ld, const float *__restrict__ cen,
+              const float *__restrict__ piv,
               const float *__restrict__ half, int M, uint32_t *cell, int32_t *id, int32_t *cnt) {
     __shared__ int lc[kMaxPivots];
     if (cnt)
@@ -288,7 +318,8 @@ k_cell_assign(const T *Z, int64_t n, int d, int64_t ld, const float *__restrict_
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     float z[DP];
 #pragma unroll
-    for (int t = 0; t < DP; ++t) z[t] = (t < d && i < n) ? -(float)Z[(int64_t)t * ld + i] : 0.0f;
+    for (int t = 0; t < DP; ++t)
+        z[t] = (t < d && i < n) ? -centred(Z[(int64_t)t * ld + i], cen ? cen[t] : 0.0f) : 0.0f;
     float best = __builtin_huge_valf();
     int bm = 0;
     for (int m = 0; m < M; ++m) {
@@ -350,14 +381,14 @@ k_cell_slots(const uint32_t *scell, const int32_t *sid, int64_t n, const int64_t
 }
 
 // One block per group: rows in slot order (Zs), the operands, |y|^2 and |y - z|
-// per slot (y the scaled operand value, z the scaled point), and the group's
+// per slot (y the operand value, z the centred and scaled point), and the group's
 // mean, radius and operand row.  One part: q rows [h, 1, 1, 1], candidate and
 // centre rows [h, n1, n2, n3], n1 + n2 + n3 = -|y|^2 / 2; two parts: [h, l, h,
 // 1, 1, 1] and [h, h, l, n1, n2, n3].  gmax: [0] max |y|^2 and [1] max error over
-// the points, [2] max |y|^2 over the means, [3] max |z|^2 unscaled.
+// the points, [2] max |y|^2 over the means, [3] max |z|^2 unscaled (centred).
 template <int KP, bool SPLIT, class T>
 __global__ void __launch_bounds__(kBlock)
-k_cell_prep(const T *Zr, int d, const int32_t *perm, const int *tot, uint16_t *zq,
+k_cell_prep(const T *Zr, int d, const float *cen, const int32_t *perm, const int *tot, uint16_t *zq,
             uint16_t *zc, uint16_t *zb, float *Rb, T *Zs, float *nhat, float *eps,
             unsigned *gmax) {
     __shared__ float zt[kGrp * 65];
@@ -385,7 +416,7 @@ k_cell_prep(const T *Zr, int d, const int32_t *perm, const int *tot, uint16_t *z
         const int r = e / d, t = e - r * d;
         const T z = ids[r] >= 0 ? Zr[(int64_t)ids[r] * d + t] : T(0);
         Zs[s0 * d + e] = z;
-        zt[r * ldz + t] = (float)(z * (T)sc);
+        zt[r * ldz + t] = ids[r] >= 0 ? centred(z, cen[t]) * sc : 0.0f;
     }
     __syncthreads();
     if (tid < d) {
@@ -408,7 +439,7 @@ k_cell_prep(const T *Zr, int d, const int32_t *perm, const int *tot, uint16_t *z
             nn += y * y;
             double x = (double)z;
             if constexpr (sizeof(T) == 8)  // against the double, not its FP32 rounding
-                if (tid < kGrp) x = (double)Zs[(s0 + tid) * d + t] * (double)sc;
+                if (tid < kGrp) x = (Zs[(s0 + tid) * d + t] - (double)cen[t]) * (double)sc;
             ee += (y - x) * (y - x);
             a = fmaf(z - mean[t], z - mean[t], a);
         }
@@ -427,6 +458,9 @@ k_cell_prep(const T *Zr, int d, const int32_t *perm, const int *tot, uint16_t *z
         if (live) {
             nf = (float)(nn * (1.0 + 1e-6)) + 1e-30f;
             ef = (float)(sqrt(ee) * (1.0 + 1e-6));
+            // FP32 points: z - cen was rounded (2^-24 of each coordinate)
+            if constexpr (sizeof(T) == 4)
+                if (tid < kGrp) ef += 6e-8f * sqrtf(nf);
             rad = a == a ? sqrtf(a) * (1.0f + 1e-5f) : __builtin_huge_valf();
         }
         if (tid < kGrp) {
@@ -487,9 +521,8 @@ k_cell_prep(const T *Zr, int d, const int32_t *perm, const int *tot, uint16_t *z
         atomicMax(&gmax[1], max(red[1][0], red[1][1]));
         atomicMax(&gmax[2], __float_as_uint(nf));
         float r = __uint_as_float(max(red[2][0], red[2][1])) + ef;
-        // the radius was taken of the FP32 roundings of the doubles
-        if constexpr (sizeof(T) == 8)
-            r += 1.2e-7f * sqrtf(__uint_as_float(max(red[0][0], red[0][1])));
+        // the radius was taken of FP32 roundings
+        r += 1.2e-7f * sqrtf(__uint_as_float(max(red[0][0], red[0][1])));
         Rb[g] = r * (1.0f + 1e-5f) + 1e-30f;
     }
 }
@@ -921,7 +954,7 @@ void run_cell(int64_t n, int64_t d, int64_t k, int include_self, int M, KnnWork 
     {
         ProfScope ps("knn_prep", st, 8.0 * n * d + 4.0 * n * KP);
         hipLaunchKernelGGL((k_cell_prep<KP, SPLIT, T>), dim3((unsigned)ngt), dim3(kBlock), 0, st, zr,
-                           (int)d, w.perm.get(), tot, (uint16_t *)w.zq.get(),
+                           (int)d, w.piv.get(), w.perm.get(), tot, (uint16_t *)w.zq.get(),
                            (uint16_t *)w.zc.get(), (uint16_t *)w.zcp.get(), w.scf.get(),
                            zs, w.nhat.get(), w.eps.get(), w.gmax.get());
         SEV_LAUNCH_CHECK();
@@ -978,16 +1011,16 @@ int64_t knn_cell(const T *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int in
     int M = 16;
     while (M < kMaxPivots && (int64_t)M * 1024 < n) M <<= 1;
     const int nsam = (int)std::min<int64_t>(n, kSample);
-    w.piv.ensure((size_t)(2 * kMaxPivots * kPivLd + 2 * kMaxPivots + kSample * kPivLd));
+    w.piv.ensure((size_t)(kPivLd + 2 * kMaxPivots * kPivLd + 2 * kMaxPivots + kSample * kPivLd));
     w.ctot.ensure(1);
     w.gmax.ensure(4);
-    float *piv = w.piv.get(), *pivo = piv + kMaxPivots * kPivLd,
+    float *cen = w.piv.get(), *piv = cen + kPivLd, *pivo = piv + kMaxPivots * kPivLd,
           *half = pivo + kMaxPivots * kPivLd, *halfo = half + kMaxPivots,
           *sam = halfo + kMaxPivots;
     if (!split) {
         w.ccnt.ensure(1);
-        hipLaunchKernelGGL(k_cell_sample<T>, dim3(128), dim3(kBlock), 0, st, Z, (int64_t)1, ld, n,
-                           (int)d, kTestPivots, sam, w.ccnt.get());
+        hipLaunchKernelGGL(k_cell_sample<T>, dim3(128), dim3(kBlock), 0, st, Z, (int64_t)1, ld,
+                           (const float *)nullptr, n, (int)d, kTestPivots, sam, w.ccnt.get());
         SEV_LAUNCH_CHECK();
         hipLaunchKernelGGL(k_cell_test<T>, dim3(kTestQueries), dim3(kBlock), 0, st, Z, n, (int)d,
                            ld, sam, w.ccnt.get());
@@ -999,9 +1032,11 @@ int64_t knn_cell(const T *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int in
     }
     w.zrb.ensure((size_t)(n * d) * sizeof(T));
     T *zr = (T *)w.zrb.get();
-    SEV_HIP(hipMemsetAsync(w.gmax.get(), 0, 4 * sizeof(unsigned), st));
+    hipLaunchKernelGGL(k_cell_centre<T>, dim3((unsigned)d), dim3(kBlock), 0, st, Z, n, ld, cen,
+                       w.gmax.get());
+    SEV_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_cell_rows<T>, dim3((unsigned)ceil_div(n, (int64_t)kWave)), dim3(kBlock), 0,
-                       st, Z, n, (int)d, ld, zr, w.gmax.get() + 3);
+                       st, Z, n, (int)d, ld, cen, zr, w.gmax.get() + 3);
     SEV_LAUNCH_CHECK();
     {
         ProfScope ps("knn_order", st, 4.0 * n * d + 24.0 * n);
@@ -1015,14 +1050,14 @@ int64_t knn_cell(const T *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int in
         w.perm.ensure((size_t)ns);
         SEV_HIP(hipMemsetAsync(w.ccell.get(), 0, sizeof(int32_t) * kMaxPivots, st));
         SEV_HIP(hipMemsetAsync(w.perm.get(), 0xFF, sizeof(int32_t) * (size_t)ns, st));
-        auto assign = [&](const auto *X, int64_t nx, int64_t lx, const float *pv, const float *hv,
-                          uint32_t *cell, int32_t *id, int32_t *cnt) {
+        auto assign = [&](const auto *X, int64_t nx, int64_t lx, const float *cn, const float *pv,
+                          const float *hv, uint32_t *cell, int32_t *id, int32_t *cnt) {
             auto go = [&](auto dp) {
                 constexpr int DP = decltype(dp)::value;
                 typedef std::remove_const_t<std::remove_pointer_t<decltype(X)>> TX;
                 hipLaunchKernelGGL((k_cell_assign<DP, TX>),
-                                   dim3((unsigned)ceil_div(nx, (int64_t)kBlock)), dim3(kBlock), 0, st, X, nx, (int)d, lx, pv, hv, M, cell, id,
-                                   cnt);
+                                   dim3((unsigned)ceil_div(nx, (int64_t)kBlock)), dim3(kBlock), 0, st, X, nx,
+                                   (int)d, lx, cn, pv, hv, M, cell, id, cnt);
             };
             if (d <= 16)
                 go(std::integral_constant<int, 16>());
@@ -1034,15 +1069,15 @@ int64_t knn_cell(const T *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int in
                 go(std::integral_constant<int, 64>());
             SEV_LAUNCH_CHECK();
         };
-        hipLaunchKernelGGL(k_cell_pivots<T>, dim3(64), dim3(kBlock), 0, st, zr, n, (int)d, M,
-                           piv);
+        hipLaunchKernelGGL(k_cell_pivots<T>, dim3(64), dim3(kBlock), 0, st, zr, cen, n,
+                           (int)d, M, piv);
         hipLaunchKernelGGL(k_cell_half, dim3((unsigned)ceil_div((int64_t)M, (int64_t)kBlock)),
                            dim3(kBlock), 0, st, piv, M, half);
-        hipLaunchKernelGGL(k_cell_sample<T>, dim3(256), dim3(kBlock), 0, st, zr, d, (int64_t)1, n,
-                           (int)d, nsam, sam, (int *)nullptr);
+        hipLaunchKernelGGL(k_cell_sample<T>, dim3(256), dim3(kBlock), 0, st, zr, d, (int64_t)1, cen,
+                           n, (int)d, nsam, sam, (int *)nullptr);
         SEV_LAUNCH_CHECK();
         for (int it = 0; it < 2; ++it) {
-            assign((const float *)sam, nsam, nsam, piv, half, w.skey2.get(), nullptr, nullptr);
+            assign((const float *)sam, nsam, nsam, nullptr, piv, half, w.skey2.get(), nullptr, nullptr);
             hipLaunchKernelGGL(k_cell_means, dim3((unsigned)M), dim3(kBlock), 0, st, sam, nsam,
                                (int)d, w.skey2.get(), piv, half);
             SEV_LAUNCH_CHECK();
@@ -1050,7 +1085,7 @@ int64_t knn_cell(const T *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int in
         hipLaunchKernelGGL(k_cell_order, dim3(1), dim3(kMaxPivots), 0, st, piv, half, M, (int)d,
                            pivo, halfo);
         SEV_LAUNCH_CHECK();
-        assign(Z, n, ld, pivo, halfo, w.skey.get(), w.sval.get(), w.ccell.get());
+        assign(Z, n, ld, cen, pivo, halfo, w.skey.get(), w.sval.get(), w.ccell.get());
         hipLaunchKernelGGL(k_cell_offsets, dim3(1), dim3(kMaxPivots), 0, st, w.ccell.get(), M,
                            w.coff.get(), w.coff.get() + kMaxPivots, w.ctot.get());
         SEV_LAUNCH_CHECK();

@@ -99,6 +99,24 @@ def test_cells_rows_left(sev, orc, n, d, k, include_self):
         assert 200 <= left < n // 4
 
 
+@pytest.mark.parametrize("precision,offset", [("fp32", 300.0), ("bf16", 3000.0), ("fp32", -2e4),
+                                              ("fp64", 1e6)])
+def test_cells_far_from_the_origin(sev, orc, precision, offset):
+    """Points far from the origin compared with their distances: the operands
+    are taken around their centre, so rows keep their certificates."""
+    n, d, k = 13000, 48, 15
+    X = _points(n, d, 12, seed=48).astype(np.float64 if precision == "fp64" else np.float32)
+    X[:, ::2] += X.dtype.type(offset)
+    if precision == "fp64":
+        idx, dist, left = sev.ann(X, k, return_fallback=True)
+    else:
+        idx, dist, left, ran = _search(sev, X, k, precision=precision)
+        assert "knn_cell" in ran
+    ridx, rdist = orc.knn(X, k)
+    assert np.array_equal(idx, ridx) and np.array_equal(dist, rdist)
+    assert left < n // 100
+
+
 # both sides of the lines between the searches, for points in groups and without
 @pytest.mark.parametrize("n,d,k,precision,grouped,want",
                          [(12300, 50, 20, "fp32", True, "exhaustive"),
