@@ -29,8 +29,8 @@
 // matter.
 //
 // Measured, k = 20: 1,000,000 x 50, 40 clusters, one part: 526 -> 73 ms (65 of
-// them k_knn_cell); 100,000 x 50, 24 clusters, two parts: 27.3 -> 3.6 ms;
-// 5,000 x 50: 1.68 -> 0.66 ms.  Without clusters nothing is skipped and the two
+// them k_knn_cell); 100,000 x 50, 24 clusters, two parts: 27.3 -> 3.6 ms; 20,000 x
+// 50, 12 clusters: 4.9 -> 0.86.  Without clusters nothing is skipped and the two
 // sweeps cost more than the one with insertion (1,000,000 Gaussian points: 165
 // ms by sev_knn_mfma.hip), so the 16-bit form keeps that search there; the FP32
 // form is faster this way in either case.
@@ -45,9 +45,10 @@
 //
 // A block holds 128 queries (4 wavefronts of 32) and 64-candidate tiles in
 // two LDS buffers: 80 KB at KP = 160, so two blocks share a compute unit, three
-// at KP <= 64.  Bound: the candidate rows of the needed groups, which mostly
-// come from beyond L2 (1.3 us per tile and block at KP = 160, 0.27 us of them
-// MFMA).
+// at KP <= 64.  Bound: the chain of a tile (rows from beyond L2, LDS, matrix
+// instructions, maxima), 1.3 us per tile and block at KP = 160, 0.27 us of them
+// MFMA; no unit is full (1,000,000 x 50: matrix cores 15% busy, VALU 37%, 72% of
+// the L2 requests missing, at 2.1 TB/s).
 #include "sev_kernels.hpp"
 
 #include <hipcub/hipcub.hpp>
@@ -953,8 +954,8 @@ void run_cell(int64_t n, int64_t d, int64_t k, int include_self, int M, KnnWork 
     const int *tot = w.ctot.get();
     {
         ProfScope ps("knn_prep", st, 8.0 * n * d + 4.0 * n * KP);
-        hipLaunchKernelGGL((k_cell_prep<KP, SPLIT, T>), dim3((unsigned)ngt), dim3(kBlock), 0, st, zr,
-                           (int)d, w.piv.get(), w.perm.get(), tot, (uint16_t *)w.zq.get(),
+        hipLaunchKernelGGL((k_cell_prep<KP, SPLIT, T>), dim3((unsigned)ngt), dim3(kBlock), 0, st,
+                           zr, (int)d, w.piv.get(), w.perm.get(), tot, (uint16_t *)w.zq.get(),
                            (uint16_t *)w.zc.get(), (uint16_t *)w.zcp.get(), w.scf.get(),
                            zs, w.nhat.get(), w.eps.get(), w.gmax.get());
         SEV_LAUNCH_CHECK();
@@ -1056,8 +1057,8 @@ int64_t knn_cell(const T *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int in
                 constexpr int DP = decltype(dp)::value;
                 typedef std::remove_const_t<std::remove_pointer_t<decltype(X)>> TX;
                 hipLaunchKernelGGL((k_cell_assign<DP, TX>),
-                                   dim3((unsigned)ceil_div(nx, (int64_t)kBlock)), dim3(kBlock), 0, st, X, nx,
-                                   (int)d, lx, cn, pv, hv, M, cell, id, cnt);
+                                   dim3((unsigned)ceil_div(nx, (int64_t)kBlock)), dim3(kBlock), 0,
+                                   st, X, nx, (int)d, lx, cn, pv, hv, M, cell, id, cnt);
             };
             if (d <= 16)
                 go(std::integral_constant<int, 16>());
@@ -1077,7 +1078,8 @@ int64_t knn_cell(const T *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int in
                            n, (int)d, nsam, sam, (int *)nullptr);
         SEV_LAUNCH_CHECK();
         for (int it = 0; it < 2; ++it) {
-            assign((const float *)sam, nsam, nsam, nullptr, piv, half, w.skey2.get(), nullptr, nullptr);
+            assign((const float *)sam, nsam, nsam, nullptr, piv, half, w.skey2.get(), nullptr,
+                   nullptr);
             hipLaunchKernelGGL(k_cell_means, dim3((unsigned)M), dim3(kBlock), 0, st, sam, nsam,
                                (int)d, w.skey2.get(), piv, half);
             SEV_LAUNCH_CHECK();
@@ -1143,7 +1145,8 @@ template int64_t knn_cell<float>(const float *, int64_t, int64_t, int64_t, int64
 void knn_cell_f64(const double *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int include_self,
                   KnnWork &w, int32_t *idx, double *dist, hipStream_t st, int64_t *n_fallback) {
     const int64_t nf = knn_cell<double>(Z, n, d, ld, k, include_self, true, w, idx, dist, st);
-    if (nf > 0) knn_exact_rows<double>(Z, n, d, ld, k, include_self, w.fail.get(), nf, idx, dist, st);
+    if (nf > 0)
+        knn_exact_rows<double>(Z, n, d, ld, k, include_self, w.fail.get(), nf, idx, dist, st);
     if (n_fallback) *n_fallback = nf;
 }
 

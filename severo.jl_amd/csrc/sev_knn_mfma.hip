@@ -1335,9 +1335,11 @@ void knn_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int i
     }
     if (bf16) {
         if (k <= 24 && d + 2 <= 64 && d + 1 <= 52)
-            run_mfma<1, 64, 2, 32, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback, rows);
+            run_mfma<1, 64, 2, 32, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st,
+                                       n_fallback, rows);
         else if (k <= 40 && d + 2 <= 64 && d + 1 <= 52)
-            run_mfma<1, 64, 2, 48, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback, rows);
+            run_mfma<1, 64, 2, 48, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st,
+                                       n_fallback, rows);
         else if (k <= 24 && d + 2 <= 64)
             run_mfma<1, 64, 2, 32, 128>(Z, n, d, ld, k, include_self, w, idx, dist, st,
                                         n_fallback, rows);
@@ -1348,9 +1350,11 @@ void knn_mfma(const float *Z, int64_t n, int64_t d, int64_t ld, int64_t k, int i
             run_mfma<1, 64, 1, 64, 52>(Z, n, d, ld, k, include_self, w, idx, dist, st,
                                        n_fallback, rows);
         else if (d + 2 <= 64)
-            run_mfma<1, 64, 1, 64, 0>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback, rows);
+            run_mfma<1, 64, 1, 64, 0>(Z, n, d, ld, k, include_self, w, idx, dist, st,
+                                      n_fallback, rows);
         else
-            run_mfma<1, 128, 1, 64, 0>(Z, n, d, ld, k, include_self, w, idx, dist, st, n_fallback, rows);
+            run_mfma<1, 128, 1, 64, 0>(Z, n, d, ld, k, include_self, w, idx, dist, st,
+                                       n_fallback, rows);
     } else {
         if (d + 1 <= 52) {
             if (k <= 24)

@@ -419,7 +419,8 @@ k_mod_parts(int64_t L, const u64 *wtot, double totw, double *part, int64_t m, co
     const int64_t m4 = m / kInEdges;
     for (int64_t q = (int64_t)b * kLvThreads + threadIdx.x; q < m4; q += (int64_t)nb * kLvThreads) {
         const int4 u = ((const int4 *)src)[q], v = ((const int4 *)adj)[q];
-        const ulonglong2 w0 = ((const ulonglong2 *)w)[2 * q], w1 = ((const ulonglong2 *)w)[2 * q + 1];
+        const ulonglong2 w0 = ((const ulonglong2 *)w)[2 * q];
+        const ulonglong2 w1 = ((const ulonglong2 *)w)[2 * q + 1];
         const int a0 = c[u.x], a1 = c[u.y], a2 = c[u.z], a3 = c[u.w];
         const int b0 = c[v.x], b1 = c[v.y], b2 = c[v.z], b3 = c[v.w];
         s += (a0 == b0 ? w0.x : 0) + (a1 == b1 ? w0.y : 0);
@@ -1047,9 +1048,9 @@ struct Louvain {
         k_fill_u64<<<grid_of(ne), kLvThreads, 0, st>>>(r.w.get(), ne, 0);
         k_fill_i32<<<grid_of(nc), kLvThreads, 0, st>>>(rowcnt.get(), nc, 0);
         k_fill_u64<<<1, 1, 0, st>>>(acc.get(), 1, 0);
-        k_run_emit<<<std::min<unsigned>(kEmitBlocks, grid_of(m)), kLvThreads, 0, st>>>(m, key2.get(), val2.get(), b, flag.get(),
-                                                      pos.get(), r.adj.get(), r.src.get(),
-                                                      r.w.get(), rowcnt.get(), acc.get());
+        k_run_emit<<<std::min<unsigned>(kEmitBlocks, grid_of(m)), kLvThreads, 0, st>>>(
+            m, key2.get(), val2.get(), b, flag.get(), pos.get(), r.adj.get(), r.src.get(),
+            r.w.get(), rowcnt.get(), acc.get());
         SEV_LAUNCH_CHECK();
         u64 self = 0;
         SEV_HIP(hipMemcpyAsync(&self, acc.get(), sizeof self, hipMemcpyDeviceToHost, st));
@@ -1103,7 +1104,8 @@ int64_t louvain_cluster(int64_t n, const int64_t *colptr_d, const int32_t *row_d
                                                           val64.get());
             val_d = val64.get();
         }
-        k_max_bits<<<std::min<unsigned>(kMaxBlocks, grid_of(nnz)), kLvThreads, 0, st>>>(nnz, val_d, mx.get());
+        k_max_bits<<<std::min<unsigned>(kMaxBlocks, grid_of(nnz)), kLvThreads, 0, st>>>(
+            nnz, val_d, mx.get());
         SEV_LAUNCH_CHECK();
         SEV_HIP(hipMemcpyAsync(&maxbits, mx.get(), sizeof maxbits, hipMemcpyDeviceToHost, st));
         SEV_HIP(hipStreamSynchronize(st));

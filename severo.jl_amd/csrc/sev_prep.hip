@@ -272,8 +272,8 @@ k_gather_copy(const int64_t *feat, const int64_t *colptr, const int32_t *row, co
 //  - the quotient delta / T(count) by Markstein's correction step (below), five
 //    dependent operations with the addition to mu, instead of a division;
 //  - the 64 values of a chunk, their counts and the counts' reciprocals are
-//    made by the lanes in parallel and put in LDS, from where groups of 8
-//    steps take them ahead of the chain (readlane into scalar registers
+//    made by the lanes in parallel and put in LDS, from where groups of 8 steps
+//    (FP64: 4) take them ahead of the chain (readlane into scalar registers
 //    stalled it: 83 cycles per step in FP32, now 45; in FP64 with the division
 //    300, now 112);
 //  - whether a quotient could leave the normal range is decided per chunk, from
