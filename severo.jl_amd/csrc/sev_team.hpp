@@ -5,8 +5,8 @@
 #include <cstdint>
 #include <functional>
 #include <mutex>
-#include <system_error>
 #include <thread>
+#include <utility>
 #include <vector>
 
 namespace sev {
@@ -23,7 +23,7 @@ class ChunkTeam {
         th_.reserve((size_t)want);
         try {
             for (int t = 0; t < want; ++t) th_.emplace_back([this, t] { work(t); });
-        } catch (const std::system_error &) {
+        } catch (...) {  // go on with those that run
         }
         // read by the threads only once a chunk is ready
         for (int &x : left_) x = (int)th_.size();

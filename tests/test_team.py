@@ -15,6 +15,7 @@ PROGRAM = r"""
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
+#include <system_error>
 
 static int allowed;
 
